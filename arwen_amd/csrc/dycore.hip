@@ -20,6 +20,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -2987,6 +2988,8 @@ int32_t ARW_API(ensemble_create)(const Dom* members, int32_t n,
                 b.start = (const int*)(dev + off[g].start[k]);
                 b.total = off[g].total[k];
                 b.tile = k == BK_COLT ? col_tile : 256;
+                b.nz = 0;
+                for (int m : gm[g]) b.nz = std::max(b.nz, (int)members[m].nz);
             }
         }
     }

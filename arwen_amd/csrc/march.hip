@@ -217,21 +217,6 @@ struct RowSeg {
     bool live;
 };
 
-// Row segment of workgroup (blockIdx.x - first) of a grid whose first
-// `first` workgroups (a multiple of ARW_NXCD) do other work.
-__device__ __forceinline__ RowSeg row_seg_from(int nx, int ny, int first)
-{
-    const int nbx = (nx + 63) / 64;
-    const int n = (int)gridDim.x - first, b = (int)blockIdx.x - first;
-    const int L = (b % ARW_NXCD) * (n / ARW_NXCD) + b / ARW_NXCD;
-    const int by = L / nbx, bx = L - by * nbx;
-    RowSeg r;
-    r.i = bx * 64 + (int)threadIdx.x;
-    r.j = __builtin_amdgcn_readfirstlane(by * 4 + (int)threadIdx.y);
-    r.live = r.i < nx && r.j < ny;
-    return r;
-}
-
 __device__ __forceinline__ RowSeg row_seg(int nx, int ny)
 {
     const int nbx = (nx + 63) / 64;
@@ -254,6 +239,25 @@ __device__ __forceinline__ RowSeg row_seg_at(int nx, int ny, int L)
     r.j = __builtin_amdgcn_readfirstlane(by * 4 + (int)threadIdx.y);
     r.live = r.i < nx && r.j < ny;
     return r;
+}
+
+// Level groups.  gridDim.y splits the levels of a column march into equal
+// groups, workgroup blockIdx.y marching levels [k0, k1): at few columns one
+// march per column leaves most SIMDs with a single wave or none, waiting on
+// one level's loads at a time.  A group whose k0 is past the end is empty
+// (its waves return at once).
+struct Levels {
+    int k0, k1;
+};
+
+__device__ __forceinline__ Levels level_group(int nz)
+{
+    const int n = ((int)gridDim.y > 1)
+                      ? (nz + (int)gridDim.y - 1) / (int)gridDim.y : nz;
+    Levels l;
+    l.k0 = (int)blockIdx.y * n;
+    l.k1 = l.k0 + n < nz ? l.k0 + n : nz;
+    return l;
 }
 
 static inline dim3 rowseg_grid(int nx, int ny)
@@ -996,7 +1000,6 @@ __global__ __launch_bounds__(256) void k_tend_cols(typename SRC::Arg a, Sc s)
 // Acoustic substep, part 1: u''/v'' forward step on faces
 // ---------------------------------------------------------------------------
 
-// Damped-pressure window of one column for the acoustic PGF.
 // Loads of one u''/v'' level, issued one level ahead.
 struct UvIn {
     real pA = R(0.0), oA = R(0.0), pW = R(0.0), oW = R(0.0), pS = R(0.0), oS = R(0.0);
@@ -1007,132 +1010,169 @@ struct UvIn {
     real aA = R(0.0), aW = R(0.0), aS = R(0.0);      // al'' (terrain)
     real bA = R(0.0), bW = R(0.0), bS = R(0.0);      // pb (terrain)
     real u = R(0.0), ru = R(0.0), v = R(0.0), rv = R(0.0);
+    real u2 = R(0.0), ru2 = R(0.0), v2 = R(0.0), rv2 = R(0.0);  // duplicates
 };
 
-// u'' at face (j, iu) and/or v'' at face (jv, i) through all levels
-// (reference acoustic.cu:244-314).  A is the mass column east of the u face
-// and north of the v face, W its west and S its south neighbour.  The
-// damped pressure p'' + smdiv (p'' - p''_old) rides in 4-level windows for
-// the surface and lid extrapolations of dpn.
-template <bool B3, bool USEP, bool DU, bool DV, bool SUM = false,
-          bool XO = true>
-__device__ __forceinline__ void uv_march(const Dom& d, const Sc& s, int rA,
-                                         int rS, int rU, unsigned bA,
-                                         unsigned bW, unsigned bS, unsigned bu,
-                                         unsigned bv)
+// u'' on face (j, i) and v'' on face (j, i) through a group of levels
+// (reference acoustic.cu:244-314): row-segment waves, the thread of mass
+// column (j, i).  A is that column, W its west and S its south neighbour.
+// The damped pressure p'' + smdiv (p'' - p''_old) rides in 4-level windows
+// for the surface and lid extrapolations of dpn; a group that starts above
+// the surface loads the two levels below it into its windows.
+//
+// The periodic duplicate faces (u'' at i = nx, v'' at j = ny) take the
+// pressure gradient of face 0 with their own u''/ru_t (v''/rv_t), so the
+// threads of column i = 0 (row j = 0) advance them beside their own: as
+// marches of their own they were one thread per row or column, whose
+// uncoalesced loads outlived the main work (at 192x160x50 most of the
+// launch's 155 us).
+template <class SRC, bool B3, bool USEP, bool SUM = false, bool XO = true>
+__global__ __launch_bounds__(256) void k_uv(typename SRC::Arg a, Sc s)
 {
-    const int nz = d.nz, ny = d.ny, nx = d.nx, st = ny * nx;
-    const int stu = ny * (nx + 1), stv = (ny + 1) * nx;
+    int m, g;
+    if (!SRC::locate(a, m, g)) return;
+    const Dom& d = SRC::dom(a, m);
+    const int nz = d.nz, ny = d.ny, nx = d.nx, st = ny * nx, pu = nx + 1;
+    const int stu = ny * pu, stv = (ny + 1) * nx;
+    const RowSeg rs = SRC::many ? row_seg_at(nx, ny, g) : row_seg(nx, ny);
+    const Levels lv = level_group(nz);
+    if (!rs.live || lv.k0 >= lv.k1) return;
+    const int i = rs.i, j = rs.j;
+    const int jm = (j == 0) ? ny - 1 : j - 1;
+    const int rA = j * nx, rS = jm * nx, rU = j * pu;
+    unsigned bA = RB * i, bW = RB * ((i == 0) ? nx - 1 : i - 1);
+    const unsigned bD = RB * nx;                 // duplicate u face column
+    const int rD = ny * nx;                      // duplicate v face row
+    const bool dupu = i == 0, dupv = j == 0;     // dupv: wave-uniform
     const real smdiv = s.smdiv, dtau = s.dtau;
     kreal* c1h = kview(d.c1h);
     kreal* c2h = kview(d.c2h);
     kreal* fnm = kview(d.fnm);
     kreal* fnp = kview(d.fnp);
     kreal* rdnw = kview(d.rdnw);
-    auto opaque_all = [&]() {
-        colb_opaque(bA); colb_opaque(bW); colb_opaque(bS);
-        colb_opaque(bu); colb_opaque(bv);
+    auto opaque_all = [&]() { colb_opaque(bA); colb_opaque(bW); };
+    auto pd = [&](real x, real o) {
+        real b = USEP ? o : x;
+        return x + smdiv * (x - b);
     };
-    auto pd = [&](real a, real o) {
-        real b = USEP ? o : a;
-        return a + smdiv * (a - b);
+    auto pd_at = [&](int k, int row, unsigned cb) {
+        return pd(gld(d.p_pp, k * st + row, cb),
+                  USEP ? gld(d.p_pp_old, k * st + row, cb) : R(0.0));
     };
     const real mA = gld(d.mub2d, rA, bA) + gld(d.mup, rA, bA);
-    const real muf_u = DU ? R(0.5) * ((gld(d.mub2d, rA, bW) + gld(d.mup, rA, bW)) + mA)
-                           : R(0.0);
-    const real muf_v = DV ? R(0.5) * ((gld(d.mub2d, rS, bS) + gld(d.mup, rS, bS)) + mA)
-                           : R(0.0);
+    const real muf_u = R(0.5) * ((gld(d.mub2d, rA, bW) + gld(d.mup, rA, bW)) + mA);
+    const real muf_v = R(0.5) * ((gld(d.mub2d, rS, bA) + gld(d.mup, rS, bA)) + mA);
     const real mppA = gld(d.mu_pp, rA, bA);
-    const real dmu_u = DU ? gld(d.mu_pp, rA, bW) + mppA : R(0.0);
-    const real dmu_v = DV ? gld(d.mu_pp, rS, bS) + mppA : R(0.0);
+    const real dmu_u = gld(d.mu_pp, rA, bW) + mppA;
+    const real dmu_v = gld(d.mu_pp, rS, bA) + mppA;
 
     // windows S(k-2), S(k-1), S(k), S(k+1) of the damped pressure
     opaque_all();
-    real pa[4] = {R(0.0), R(0.0), R(0.0), R(0.0)}, pw[4] = {R(0.0), R(0.0), R(0.0), R(0.0)};
-    real ps[4] = {R(0.0), R(0.0), R(0.0), R(0.0)};
-    pa[2] = pd(gld(d.p_pp, 0 + rA, bA), gld(d.p_pp_old, 0 + rA, bA));
-    pa[3] = pd(gld(d.p_pp, st + rA, bA), gld(d.p_pp_old, st + rA, bA));
-    const real pa2 = pd(gld(d.p_pp, 2 * st + rA, bA), gld(d.p_pp_old, 2 * st + rA, bA));
-    real dnu_0 = R(0.0), dnv_0 = R(0.0);
-    if (DU) {
-        pw[2] = pd(gld(d.p_pp, 0 + rA, bW), gld(d.p_pp_old, 0 + rA, bW));
-        pw[3] = pd(gld(d.p_pp, st + rA, bW), gld(d.p_pp_old, st + rA, bW));
-        const real pw2 = pd(gld(d.p_pp, 2 * st + rA, bW), gld(d.p_pp_old, 2 * st + rA, bW));
-        real S0 = pa[2] + pw[2], S1 = pa[3] + pw[3], S2 = pa2 + pw2;
-        dnu_0 = R(0.5) * ((d.cf1 * S0 + d.cf2 * S1) + d.cf3 * S2);
-    }
-    if (DV) {
-        ps[2] = pd(gld(d.p_pp, 0 + rS, bS), gld(d.p_pp_old, 0 + rS, bS));
-        ps[3] = pd(gld(d.p_pp, st + rS, bS), gld(d.p_pp_old, st + rS, bS));
-        const real ps2 = pd(gld(d.p_pp, 2 * st + rS, bS), gld(d.p_pp_old, 2 * st + rS, bS));
-        real S0 = pa[2] + ps[2], S1 = pa[3] + ps[3], S2 = pa2 + ps2;
+    const int k0 = lv.k0, kp1 = k0 + 1 < nz ? k0 + 1 : nz - 1;
+    real pa[4] = {R(0.0), R(0.0), pd_at(k0, rA, bA), pd_at(kp1, rA, bA)};
+    real pw[4] = {R(0.0), R(0.0), pd_at(k0, rA, bW), pd_at(kp1, rA, bW)};
+    real ps[4] = {R(0.0), R(0.0), pd_at(k0, rS, bA), pd_at(kp1, rS, bA)};
+    real dnu_0, dnv_0;
+    if (k0 == 0) {
+        const real pa2 = pd_at(2, rA, bA);
+        {
+            real S0 = pa[2] + pw[2], S1 = pa[3] + pw[3];
+            real S2 = pa2 + pd_at(2, rA, bW);
+            dnu_0 = R(0.5) * ((d.cf1 * S0 + d.cf2 * S1) + d.cf3 * S2);
+        }
+        real S0 = pa[2] + ps[2], S1 = pa[3] + ps[3];
+        real S2 = pa2 + pd_at(2, rS, bA);
         dnv_0 = R(0.5) * ((d.cf1 * S0 + d.cf2 * S1) + d.cf3 * S2);
+    } else {
+        const int km2 = k0 >= 2 ? k0 - 2 : 0;
+        pa[1] = pd_at(k0 - 1, rA, bA);
+        pw[1] = pd_at(k0 - 1, rA, bW);
+        ps[1] = pd_at(k0 - 1, rS, bA);
+        pa[0] = pd_at(km2, rA, bA);
+        pw[0] = pd_at(km2, rA, bW);
+        ps[0] = pd_at(km2, rS, bA);
+        dnu_0 = R(0.5) * (fnm[k0] * (pa[2] + pw[2]) + fnp[k0] * (pa[1] + pw[1]));
+        dnv_0 = R(0.5) * (fnm[k0] * (pa[2] + ps[2]) + fnp[k0] * (pa[1] + ps[1]));
     }
-    real phA0 = gld(d.ph_pp, 0 + rA, bA), hpA0 = gld(d.php, 0 + rA, bA);
-    real phW0 = DU ? gld(d.ph_pp, 0 + rA, bW) : R(0.0), hpW0 = DU ? gld(d.php, 0 + rA, bW) : R(0.0);
-    real phS0 = DV ? gld(d.ph_pp, 0 + rS, bS) : R(0.0), hpS0 = DV ? gld(d.php, 0 + rS, bS) : R(0.0);
-    real gbA0 = B3 ? gld(d.phb, 0 + rA, bA) : R(0.0);
-    real gbW0 = (B3 && DU) ? gld(d.phb, 0 + rA, bW) : R(0.0);
-    real gbS0 = (B3 && DV) ? gld(d.phb, 0 + rS, bS) : R(0.0);
+    const int w0 = k0 * st;
+    real phA0 = gld(d.ph_pp, w0 + rA, bA), hpA0 = gld(d.php, w0 + rA, bA);
+    real phW0 = gld(d.ph_pp, w0 + rA, bW), hpW0 = gld(d.php, w0 + rA, bW);
+    real phS0 = gld(d.ph_pp, w0 + rS, bA), hpS0 = gld(d.php, w0 + rS, bA);
+    real gbA0 = B3 ? gld(d.phb, w0 + rA, bA) : R(0.0);
+    real gbW0 = B3 ? gld(d.phb, w0 + rA, bW) : R(0.0);
+    real gbS0 = B3 ? gld(d.phb, w0 + rS, bA) : R(0.0);
 
     auto load = [&](UvIn& L, int k) {
         const unsigned lp = (k + 2 < nz ? k + 2 : nz - 1) * st;
         const unsigned lw = (k + 1) * st, lm = k * st;
         L.pA = gld(d.p_pp, lp + rA, bA);
-        if (USEP) L.oA = gld(d.p_pp_old, lp + rA, bA);
+        L.pW = gld(d.p_pp, lp + rA, bW);
+        L.pS = gld(d.p_pp, lp + rS, bA);
+        if (USEP) {
+            L.oA = gld(d.p_pp_old, lp + rA, bA);
+            L.oW = gld(d.p_pp_old, lp + rA, bW);
+            L.oS = gld(d.p_pp_old, lp + rS, bA);
+        }
         L.phA = gld(d.ph_pp, lw + rA, bA);
+        L.phW = gld(d.ph_pp, lw + rA, bW);
+        L.phS = gld(d.ph_pp, lw + rS, bA);
         L.hpA = gld(d.php, lw + rA, bA);
+        L.hpW = gld(d.php, lw + rA, bW);
+        L.hpS = gld(d.php, lw + rS, bA);
         L.altA = gld(d.alt, lm + rA, bA);
+        L.altW = gld(d.alt, lm + rA, bW);
+        L.altS = gld(d.alt, lm + rS, bA);
         if (B3) {
             L.gbA = gld(d.phb, lw + rA, bA);
+            L.gbW = gld(d.phb, lw + rA, bW);
+            L.gbS = gld(d.phb, lw + rS, bA);
             L.aA = gld(d.al_pp, lm + rA, bA);
+            L.aW = gld(d.al_pp, lm + rA, bW);
+            L.aS = gld(d.al_pp, lm + rS, bA);
             L.bA = gld(d.pb, lm + rA, bA);
+            L.bW = gld(d.pb, lm + rA, bW);
+            L.bS = gld(d.pb, lm + rS, bA);
         }
-        if (DU) {
-            L.pW = gld(d.p_pp, lp + rA, bW);
-            if (USEP) L.oW = gld(d.p_pp_old, lp + rA, bW);
-            L.phW = gld(d.ph_pp, lw + rA, bW);
-            L.hpW = gld(d.php, lw + rA, bW);
-            L.altW = gld(d.alt, lm + rA, bW);
-            if (B3) {
-                L.gbW = gld(d.phb, lw + rA, bW);
-                L.aW = gld(d.al_pp, lm + rA, bW);
-                L.bW = gld(d.pb, lm + rA, bW);
-            }
-            L.u = gld(d.u_pp, k * stu + rU, bu);
-            L.ru = gld(d.ru_t, k * stu + rU, bu);
+        L.u = gld(d.u_pp, k * stu + rU, bA);
+        L.ru = gld(d.ru_t, k * stu + rU, bA);
+        L.v = gld(d.v_pp, k * stv + rA, bA);
+        L.rv = gld(d.rv_t, k * stv + rA, bA);
+        if (dupu) {
+            L.u2 = gld(d.u_pp, k * stu + rU, bD);
+            L.ru2 = gld(d.ru_t, k * stu + rU, bD);
         }
-        if (DV) {
-            L.pS = gld(d.p_pp, lp + rS, bS);
-            if (USEP) L.oS = gld(d.p_pp_old, lp + rS, bS);
-            L.phS = gld(d.ph_pp, lw + rS, bS);
-            L.hpS = gld(d.php, lw + rS, bS);
-            L.altS = gld(d.alt, lm + rS, bS);
-            if (B3) {
-                L.gbS = gld(d.phb, lw + rS, bS);
-                L.aS = gld(d.al_pp, lm + rS, bS);
-                L.bS = gld(d.pb, lm + rS, bS);
-            }
-            L.v = gld(d.v_pp, k * stv + rA, bv);
-            L.rv = gld(d.rv_t, k * stv + rA, bv);
+        if (dupv) {
+            L.v2 = gld(d.v_pp, k * stv + rD, bA);
+            L.rv2 = gld(d.rv_t, k * stv + rD, bA);
+        }
+    };
+    // one face: the forward step, the sumflux sum; x, rt: its u''/v'' and
+    // slow tendency, dpxy: the pressure gradient before moist_cq's factor
+    auto advance = [&](real* pp, real* acc, const real* cq, int lev,
+                       unsigned cb, real x, real rt, real dpxy) {
+        if (XO && s.cq) dpxy = gld(cq, lev, cb) * dpxy;
+        const real n = x + dtau * (rt - dpxy);
+        gst(pp, lev, cb, n);
+        if (SUM) {
+            const real o = (s.sum == 1) ? R(0.0) : gld(acc, lev, cb);
+            gst(acc, lev, cb, o + n);
         }
     };
 
     UvIn nxt;
-    load(nxt, 0);
+    load(nxt, k0);
     auto level = [&](int k, auto last_kind) {
         constexpr bool LAST = decltype(last_kind)::value;
         opaque_all();
         const UvIn L = nxt;
-        if (!LAST) load(nxt, k + 1);
+        if (!LAST && k + 1 < lv.k1) load(nxt, k + 1);
         const real c1 = c1h[k], c2 = c2h[k];
-        const real phA1 = L.phA, hpA1 = L.hpA, gbA1 = L.gbA;
-        const real altA = L.altA;
+        const int lu = k * stu + rU, lvv = k * stv;
         auto dn_top = [&](real Sk, real Sm1, real Sm2) {
             return s.top_lid ? R(0.5) * ((d.cf1 * Sk + d.cf2 * Sm1) + d.cf3 * Sm2)
                              : R(0.0);
         };
-        if (DU) {
+        {
             real Sk = pa[2] + pw[2];
             real dn_up;
             if (LAST) {
@@ -1141,28 +1181,22 @@ __device__ __forceinline__ void uv_march(const Dom& d, const Sc& s, int rA,
                 real Sp = pa[3] + pw[3];
                 dn_up = R(0.5) * (fnm[k + 1] * Sp + fnp[k + 1] * Sk);
             }
-            real dph = (phA1 - L.phW) + (phA0 - phW0);
+            real dph = (L.phA - L.phW) + (phA0 - phW0);
             real dpe = pa[2] - pw[2];
-            real brk = dph + (altA + L.altW) * dpe;
+            real brk = dph + (L.altA + L.altW) * dpe;
             if (B3) brk = brk + (L.aA + L.aW) * (L.bA - L.bW);
             real dpxy = ((R(0.5) * s.rdx) * (c1 * muf_u + c2)) * brk;
-            real phsA = hpA0 + hpA1, phsB = hpW0 + L.hpW;
+            real phsA = hpA0 + L.hpA, phsB = hpW0 + L.hpW;
             real dphp = R(0.5) * (phsA - phsB);
-            if (B3) dphp = dphp + R(0.5) * ((gbA0 + gbA1) - (gbW0 + L.gbW));
+            if (B3) dphp = dphp + R(0.5) * ((gbA0 + L.gbA) - (gbW0 + L.gbW));
             dpxy = dpxy + (s.rdx * dphp) * (rdnw[k] * (dn_up - dnu_0)
                                             - (R(0.5) * c1) * dmu_u);
-            if (XO && s.cq) dpxy = gld(d.cqu, k * stu + rU, bu) * dpxy;   // moist_cq
-            const real un = L.u + dtau * (L.ru - dpxy);
-            gst(d.u_pp, k * stu + rU, bu, un);
-            if (SUM) {
-                const real acc = (s.sum == 1) ? R(0.0)
-                                              : gld(d.ru_m, k * stu + rU, bu);
-                gst(d.ru_m, k * stu + rU, bu, acc + un);
-            }
+            advance(d.u_pp, d.ru_m, d.cqu, lu, bA, L.u, L.ru, dpxy);
+            if (dupu) advance(d.u_pp, d.ru_m, d.cqu, lu, bD, L.u2, L.ru2, dpxy);
             dnu_0 = dn_up;
             phW0 = L.phW; hpW0 = L.hpW; gbW0 = L.gbW;
         }
-        if (DV) {
+        {
             real Sk = pa[2] + ps[2];
             real dn_up;
             if (LAST) {
@@ -1171,83 +1205,34 @@ __device__ __forceinline__ void uv_march(const Dom& d, const Sc& s, int rA,
                 real Sp = pa[3] + ps[3];
                 dn_up = R(0.5) * (fnm[k + 1] * Sp + fnp[k + 1] * Sk);
             }
-            real dph = (phA1 - L.phS) + (phA0 - phS0);
+            real dph = (L.phA - L.phS) + (phA0 - phS0);
             real dpe = pa[2] - ps[2];
-            real brk = dph + (altA + L.altS) * dpe;
+            real brk = dph + (L.altA + L.altS) * dpe;
             if (B3) brk = brk + (L.aA + L.aS) * (L.bA - L.bS);
             real dpxy = ((R(0.5) * s.rdy) * (c1 * muf_v + c2)) * brk;
-            real phsA = hpA0 + hpA1, phsB = hpS0 + L.hpS;
+            real phsA = hpA0 + L.hpA, phsB = hpS0 + L.hpS;
             real dphp = R(0.5) * (phsA - phsB);
-            if (B3) dphp = dphp + R(0.5) * ((gbA0 + gbA1) - (gbS0 + L.gbS));
+            if (B3) dphp = dphp + R(0.5) * ((gbA0 + L.gbA) - (gbS0 + L.gbS));
             dpxy = dpxy + (s.rdy * dphp) * (rdnw[k] * (dn_up - dnv_0)
                                             - (R(0.5) * c1) * dmu_v);
-            if (XO && s.cq) dpxy = gld(d.cqv, k * stv + rA, bv) * dpxy;   // moist_cq
-            const real vn = L.v + dtau * (L.rv - dpxy);
-            gst(d.v_pp, k * stv + rA, bv, vn);
-            if (SUM) {
-                const real acc = (s.sum == 1) ? R(0.0)
-                                              : gld(d.rv_m, k * stv + rA, bv);
-                gst(d.rv_m, k * stv + rA, bv, acc + vn);
-            }
+            advance(d.v_pp, d.rv_m, d.cqv, lvv + rA, bA, L.v, L.rv, dpxy);
+            if (dupv) advance(d.v_pp, d.rv_m, d.cqv, lvv + rD, bA, L.v2, L.rv2, dpxy);
             dnv_0 = dn_up;
             phS0 = L.phS; hpS0 = L.hpS; gbS0 = L.gbS;
         }
-        phA0 = phA1; hpA0 = hpA1; gbA0 = gbA1;
+        phA0 = L.phA; hpA0 = L.hpA; gbA0 = L.gbA;
         // advance the damped-pressure windows to k+1 (level k+2 enters)
-        const bool in = k + 2 < nz;
         pa[0] = pa[1]; pa[1] = pa[2]; pa[2] = pa[3];
+        pw[0] = pw[1]; pw[1] = pw[2]; pw[2] = pw[3];
+        ps[0] = ps[1]; ps[1] = ps[2]; ps[2] = ps[3];
+        const bool in = k + 2 < nz;
         pa[3] = in ? pd(L.pA, L.oA) : R(0.0);
-        if (DU) {
-            pw[0] = pw[1]; pw[1] = pw[2]; pw[2] = pw[3];
-            pw[3] = in ? pd(L.pW, L.oW) : R(0.0);
-        }
-        if (DV) {
-            ps[0] = ps[1]; ps[1] = ps[2]; ps[2] = ps[3];
-            ps[3] = in ? pd(L.pS, L.oS) : R(0.0);
-        }
+        pw[3] = in ? pd(L.pW, L.oW) : R(0.0);
+        ps[3] = in ? pd(L.pS, L.oS) : R(0.0);
     };
-    for (int k = 0; k < nz - 1; ++k) level(k, std::false_type{});
-    level(nz - 1, std::true_type{});
-}
-
-// One launch: the first ne workgroups advance the periodic duplicate faces
-// (u'' at i = nx, one per row; v'' at j = ny, one per column; each with its
-// own u''/ru_t and the PGF of face 0), dispatched first so they overlap the
-// main work; the rest are row-segment waves in which the thread of mass
-// column (j, i) advances u'' on face (j, i) and v'' on face (j, i).
-// Batched (Many): each member's logical range holds its edge workgroups
-// first; ne_arg is unused.
-template <class SRC, bool B3, bool USEP, bool SUM = false, bool XO = true>
-__global__ __launch_bounds__(256) void k_uv(typename SRC::Arg a, Sc s, int ne_arg)
-{
-    int m, g;
-    if (!SRC::locate(a, m, g)) return;
-    const Dom& d = SRC::dom(a, m);
-    const int ny = d.ny, nx = d.nx, pu = nx + 1;
-    const int ne = SRC::many ? (ny + nx + 255) / 256 : ne_arg;
-    if (g < ne) {
-        const int t = g * 256 + threadIdx.y * 64 + threadIdx.x;
-        if (t < ny) {
-            const int j = t;
-            uv_march<B3, USEP, true, false, SUM, XO>(
-                d, s, 0, 0, 0, RB * (j * nx), RB * (j * nx + nx - 1), 0u,
-                RB * (j * pu + nx), 0u);
-        } else if (t < ny + nx) {
-            const int i = t - ny;
-            uv_march<B3, USEP, false, true, SUM, XO>(
-                d, s, 0, 0, 0, RB * i, 0u, RB * ((ny - 1) * nx + i), 0u,
-                RB * (ny * nx + i));
-        }
-        return;
-    }
-    const RowSeg rs = SRC::many ? row_seg_at(nx, ny, g - ne)
-                              : row_seg_from(nx, ny, ne);
-    if (!rs.live) return;
-    const int i = rs.i, j = rs.j;
-    const int jm = (j == 0) ? ny - 1 : j - 1;
-    const unsigned bc = RB * i, bw = RB * ((i == 0) ? nx - 1 : i - 1);
-    uv_march<B3, USEP, true, true, SUM, XO>(d, s, j * nx, jm * nx, j * pu, bc, bw, bc,
-                                   bc, bc);
+    const int kb = lv.k1 < nz ? lv.k1 : nz - 1;
+    for (int k = k0; k < kb; ++k) level(k, std::false_type{});
+    if (lv.k1 == nz) level(nz - 1, std::true_type{});
 }
 
 // ---------------------------------------------------------------------------
@@ -2512,17 +2497,40 @@ hipError_t run_tend_cols(const Dom& d, const Sc& s, hipStream_t st)
     return hipGetLastError();
 }
 
+// Level groups of a launch of `blocks` 256-thread workgroups, each group at
+// least `least` levels: enough workgroups that every CU of the 256 holds
+// about `fill` of them.
+static inline unsigned level_groups(unsigned blocks, int nz, int fill,
+                                    int least)
+{
+    const unsigned most = (unsigned)(nz / least > 1 ? nz / least : 1);
+    const unsigned want = (256u * fill + blocks - 1) / (blocks ? blocks : 1);
+    return want < 1 ? 1 : (want > most ? most : want);
+}
+
+// k_uv: groups down to 2 levels, 16 workgroups a CU.  Before the groups and
+// with the duplicate faces as marches of their own a launch took 185 us at
+// 250x200x49 over terrain, 155 us at 192x160x50 moist and 38 us at 512x1x64;
+// after, 24, 19 and 8 us.  Unsplit (one group, duplicates folded) 250x200x49
+// runs 2.16 ms a step against 2.11, an ensemble of ten 96..256-wide members
+// 14.35 against 14.02, and 1000x1000x50 (two groups by this rule) 20.37
+// against 20.27; 4 levels at least instead of 2 costs 512x1x64 12 us a step.
+static unsigned uv_groups(unsigned blocks, int nz)
+{
+    return level_groups(blocks, nz, 16, 2);
+}
+
 template <bool B3, bool USEP, bool XO>
 static void launch_uv(const Dom& d, const Sc& s, hipStream_t st)
 {
-    const int ne = (int)xcd_grid((unsigned)((d.ny + d.nx + 255) / 256));
-    const dim3 g(rowseg_grid(d.nx, d.ny).x + ne);
+    dim3 g = rowseg_grid(d.nx, d.ny);
+    g.y = uv_groups(g.x, d.nz);
     if (s.sum)
         hipLaunchKernelGGL((k_uv<One, B3, USEP, true, XO>), g, dim3(64, 4), 0,
-                           st, d, s, ne);
+                           st, d, s);
     else
         hipLaunchKernelGGL((k_uv<One, B3, USEP, false, XO>), g, dim3(64, 4), 0,
-                           st, d, s, ne);
+                           st, d, s);
 }
 
 hipError_t run_uv(const Dom& d, const Sc& s, hipStream_t st)
@@ -2664,7 +2672,6 @@ int batch_blocks(const Dom& d, int kind, int col_tile)
     case BK_COLS: return (d.ny * d.nx + 255) / 256;
     case BK_COLT: return (d.ny * d.nx + col_tile - 1) / col_tile;
     case BK_ROWS: return rows;
-    case BK_UV: return (d.ny + d.nx + 255) / 256 + rows;
     case BK_TFE: return (d.nz * d.ny + d.nz * d.nx + 255) / 256;
     default: return (d.ny + d.nx + 255) / 256;
     }
@@ -2719,17 +2726,19 @@ hipError_t run_tend_cols_b(const BatchSet& b, const Sc& s, bool b3,
 
 hipError_t run_uv_b(const BatchSet& b, const Sc& s, bool b3, hipStream_t st)
 {
-    const Batch& r = b.k[BK_UV];
-    const dim3 g = bgrid(r), blk(64, 4);
+    const Batch& r = b.k[BK_ROWS];
+    dim3 g = bgrid(r);
+    const dim3 blk(64, 4);
+    g.y = uv_groups(g.x, r.nz);
     const bool usep = s.use_pold != 0;
     if (b3 && usep)
-        hipLaunchKernelGGL((k_uv<Many, true, true>), g, blk, 0, st, r, s, 0);
+        hipLaunchKernelGGL((k_uv<Many, true, true>), g, blk, 0, st, r, s);
     else if (b3)
-        hipLaunchKernelGGL((k_uv<Many, true, false>), g, blk, 0, st, r, s, 0);
+        hipLaunchKernelGGL((k_uv<Many, true, false>), g, blk, 0, st, r, s);
     else if (usep)
-        hipLaunchKernelGGL((k_uv<Many, false, true>), g, blk, 0, st, r, s, 0);
+        hipLaunchKernelGGL((k_uv<Many, false, true>), g, blk, 0, st, r, s);
     else
-        hipLaunchKernelGGL((k_uv<Many, false, false>), g, blk, 0, st, r, s, 0);
+        hipLaunchKernelGGL((k_uv<Many, false, false>), g, blk, 0, st, r, s);
     return hipGetLastError();
 }
 

@@ -1,0 +1,60 @@
+"""The step's kernels where their launches change shape: one-column and
+ragged domains, the fewest levels, remainders of the level groups and of
+the 64-column tiles, and duplicate faces that differ from face 0.  One step,
+bit-identical to the float32 oracle."""
+import numpy as np
+import pytest
+
+from helpers import DIAG, PROG, compare, oracle_and_gpu
+from oracle import dycore_np as O
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 1, 3), (5, 3, 3), (64, 4, 4), (65, 5, 7), (130, 1, 33),
+         (63, 9, 50), (200, 67, 17), (257, 60, 65), (3, 70, 130)]
+
+
+def _noisy(case, seed=5):
+    """w noise, and duplicate faces of their own (the step carries them
+    separately)."""
+    rng = np.random.default_rng(seed)
+    f = case.fields
+    f["w"][1:-1] = 0.2 * rng.standard_normal(f["w"][1:-1].shape)
+    f["u"][..., -1] += 0.05
+    f["v"][:, -1] -= 0.05
+    return case
+
+
+def _case(kind, nx, ny, nz):
+    from arwen_amd import cases as C
+    if kind == "flat":
+        return _noisy(C.ensemble_member(nx, ny, nz, seed=3))
+    if kind == "terrain":
+        return _noisy(C.stratified_hill(nx=nx, ny=ny, nz=nz, dx=3000.0,
+                                        dt=12.0, radius=20000.0,
+                                        hill=300.0))
+    if kind == "moist":
+        return _noisy(C.mixed_phase(10, nx=nx, ny=ny, nz=nz))
+    case = _noisy(C.ensemble_member(nx, ny, nz, seed=3))
+    case.cfg = case.cfg.with_(khdif=75.0, kvdif=75.0, time_step_sound=6)
+    return case
+
+
+@pytest.mark.parametrize("kind", ["flat", "terrain", "diffusion", "moist"])
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s)))
+def test_step_is_bit_identical_at_the_edges_of_the_launch_shapes(kind, size):
+    from arwen_amd import dycore
+    case = _case(kind, *size)
+    o, g = oracle_and_gpu(case)
+    names = PROG + DIAG
+    if kind == "moist":
+        import torch
+        q = ("qv", "qc", "qr") + o.extra
+        names = names + q
+        for n in q + ("h_diabatic",):
+            getattr(g, n).copy_(torch.as_tensor(getattr(o, n)))
+    O.step(o, case.cfg)
+    dycore.step(g, case.cfg)
+    for n, (err, same) in compare(o, g, names).items():
+        assert np.all(np.isfinite(getattr(o, n))), n
+        assert same == 1.0, f"{n}: rel {err:.3e}, {same:.6f} identical"
