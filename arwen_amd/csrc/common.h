@@ -65,6 +65,8 @@ struct Sc {
     // held mixing tendencies (d.d6_*) join the stage tendencies as they are
     // stored (arw_step only)
     int held;
+    // k_column_tile: rows its LDS arrays are sized for, level groups
+    int lds_rows, lds_groups;
 };
 
 static inline Sc make_sc(const arw_params* p, double dtau, int first)
@@ -98,6 +100,7 @@ static inline Sc make_sc(const arw_params* p, double dtau, int first)
     s.h5 = p->h_sca_adv_order == 5;
     s.cq = p->moist_cq != 0;
     s.held = 0;
+    s.lds_rows = s.lds_groups = 0;
     return s;
 }
 

@@ -1709,6 +1709,531 @@ __global__ __launch_bounds__(256) void k_column(typename SRC::Arg a, Sc s,
     dn_level(0, Kind<LV_LAST>{});
 }
 
+// The same substep half for a tile of TX columns by a workgroup (TX, NG):
+// level group v takes the up to L levels [k0, k1), so many levels' loads are
+// in flight at once, and only what is a recurrence runs level after level,
+// out of LDS:
+//   1. each group forms its levels' u''/v'' divergence (to LDS) and the
+//      horizontal theta flux;
+//   2. the first group sums its columns' divergence in level order (mu'') and
+//      runs the Omega'' recurrence;
+//   3. theta'', the phi'' right-hand side and the rows of the implicit
+//      system; what a group needs of the levels next to its own is exchanged
+//      through LDS, and its first and last rows follow after that;
+//   4. the first group eliminates and back-substitutes all rows from LDS
+//      (the factors too on a stage's first substep; later ones read gamma
+//      from d.gam, so alpha is formed in step 3, without the chain of
+//      divisions);
+//   5. w'', the damper, phi'' and p'' of the group's levels.
+// Each value is the expression of k_column in its order, so the two kernels
+// are bit-identical.  Alone on its CU a tile of 64 levels takes 11 us: 2 for
+// each of the two rounds of loads, 1.6 for step 2, 2 each for the divisions
+// of steps 3 and 5, 2.3 for step 4.  Loading step 3's inputs ahead of step 2
+// took 142-166 VGPRs (3 waves a SIMD instead of 4) and was slower.
+// LDS: per row and column the four values (right-hand side, then w''; gamma;
+// a; alpha), so the recurrences read a row with one instruction, between PAD
+// rows that their block reads may touch; the divergence, Omega'' and
+// column-sum arrays; the exchange; the level coefficients.
+constexpr int TILE_PAD = 8;
+enum { X_RLO, X_PLO, X_RHI, X_PHI, X_A, X_B, X_C, X_N };
+enum { CF_C1H, CF_C2H, CF_C1F, CF_C2F, CF_DNW, CF_RDNW, CF_RDN, CF_FNM, CF_FNP,
+       CF_N };
+
+template <bool B3, bool DAMP, bool AL, bool WW, bool PREC, bool XO, int TX,
+          int L>
+__global__ __launch_bounds__(512) void k_column_tile(Dom d, Sc s, real* RS pout)
+{
+    typedef typename std::conditional<PREC, double, real>::type tri;
+    constexpr int S = TX;
+    struct alignas(4 * sizeof(tri)) Row { tri w, g, a, b; };
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const int nz = d.nz, ny = d.ny, nx = d.nx, st = ny * nx;
+    const int stu = ny * (nx + 1), stv = (ny + 1) * nx;
+    const int tile = xcd_block() * TX;
+    if (tile >= st) return;                          // the whole workgroup
+    const int x = (int)threadIdx.x;
+    const int wv = (int)threadIdx.y;
+    const int nw = (int)blockDim.y;
+    // the last tile's spare lanes repeat its last column, in step with the
+    // lane that owns it
+    const int c = tile + x < st ? tile + x : st - 1;
+    const int per = (nz + s.lds_groups - 1) / s.lds_groups;
+    const int k0 = wv * per < nz ? wv * per : nz;
+    const int k1 = k0 + per < nz ? k0 + per : nz;
+    const bool some = k0 < nz;                       // this group has levels
+    const bool top = some && k1 == nz;               // owns w level nz
+    const int j = c / nx, i = c - j * nx;
+    const int ip = (i + 1 == nx) ? 0 : i + 1, im = (i == 0) ? nx - 1 : i - 1;
+    const int jp = (j + 1 == ny) ? 0 : j + 1, jm = (j == 0) ? ny - 1 : j - 1;
+    const real eps = s.epssm, dtau = s.dtau;
+    const real one_p = R(1.0) + eps, one_m = R(1.0) - eps;
+    // per-lane byte offsets of the group's first level, and level strides
+    const unsigned sm = RB * st, su = RB * stu, sv = RB * stv;
+    const int ka = some ? k0 : nz - 1;
+    const unsigned oc = RB * c, bc = ka * sm + oc;
+    const unsigned bE = ka * sm + RB * (j * nx + ip), bW = ka * sm + RB * (j * nx + im);
+    const unsigned bN = ka * sm + RB * (jp * nx + i), bS = ka * sm + RB * (jm * nx + i);
+    const unsigned ou = RB * (j * (nx + 1) + i), bu = ka * su + ou;
+    const unsigned bv = ka * sv + oc;
+    const int cn = s.lds_rows;                       // nz + 1
+    Row* const Lr = reinterpret_cast<Row*>(lds_raw) + TILE_PAD * S + x;
+    real* const Lf = reinterpret_cast<real*>(
+        reinterpret_cast<Row*>(lds_raw) + (cn + 2 * TILE_PAD) * S);
+    real* Ldv = Lf + x;                              // divergence, Omega''
+    real* Lx = Lf + cn * S + x;                      // exchange
+    real* Lsum = Lf + (cn + X_N * s.lds_groups) * S + x;
+    real* cf = Lf + (cn + X_N * s.lds_groups + 1) * S;
+    const real *c1h = cf + CF_C1H * cn, *c2h = cf + CF_C2H * cn;
+    const real *c1f = cf + CF_C1F * cn, *c2f = cf + CF_C2F * cn;
+    const real *dnw = cf + CF_DNW * cn, *rdnw = cf + CF_RDNW * cn;
+    const real *rdn = cf + CF_RDN * cn, *fnm = cf + CF_FNM * cn;
+    const real* fnp = cf + CF_FNP * cn;
+    for (int k = wv * TX + x; k <= nz; k += TX * nw) {
+        const int h = k < nz ? k : nz - 1;
+        cf[CF_C1H * cn + k] = d.c1h[h];
+        cf[CF_C2H * cn + k] = d.c2h[h];
+        cf[CF_C1F * cn + k] = d.c1f[k];
+        cf[CF_C2F * cn + k] = d.c2f[k];
+        cf[CF_DNW * cn + k] = d.dnw[h];
+        cf[CF_RDNW * cn + k] = d.rdnw[h];
+        cf[CF_RDN * cn + k] = d.rdn[h];
+        cf[CF_FNM * cn + k] = d.fnm[h];
+        cf[CF_FNP * cn + k] = d.fnp[h];
+    }
+    // theta and phi of the level dk above (or below) offset o's
+    auto theta = [&](int k, unsigned o) {
+        return (B3 ? gld(d.thb, 0, o) : d.thb[k]) + gld(d.thp, 0, o);
+    };
+    auto phfull = [&](int k, unsigned o) {
+        return (B3 ? gld(d.phb, 0, o) : d.phb[k]) + gld(d.php, 0, o);
+    };
+
+    // 1. divergence and horizontal theta flux of the wave's levels
+    const real mut = d.mub2d[c] + d.mup[c];
+    const real mupp_old = d.mu_pp[c];
+    const real rf = d.dmdt_rf[c], rmu = d.rmu_t[c];
+    real th[L], hxy[L], dv[L];
+#pragma unroll
+    for (int q = 0; q < L; ++q) {
+        const int k = ka + q < nz ? ka + q : nz - 1;
+        const unsigned om = (k - ka) * sm, ol = (k - ka) * su, on = (k - ka) * sv;
+        const real ui = gld(d.u_pp, 0, bu + ol), uip = gld(d.u_pp, 0, bu + ol + RB);
+        const real vj = gld(d.v_pp, 0, bv + on);
+        const real vjp = gld(d.v_pp, 0, bv + on + RB * nx);
+        const real t_c = theta(k, bc + om);
+        const real te = theta(k, bE + om), tw = theta(k, bW + om);
+        const real tn = theta(k, bN + om), ts = theta(k, bS + om);
+        const real dvp = s.rdx * (uip - ui) + s.rdy * (vjp - vj);
+        dv[q] = dvp;
+        if (k0 + q < k1) Ldv[(k0 + q) * S] = d.dnw[k] * dvp;
+        const real hx = (R(0.5) * s.rdx) * (uip * (te + t_c) - ui * (t_c + tw));
+        const real hy = (R(0.5) * s.rdy) * (vjp * (tn + t_c) - vj * (t_c + ts));
+        th[q] = t_c;
+        hxy[q] = hx + hy;
+    }
+    __syncthreads();
+
+    // 2. column sum, then Omega'' (at w level k + 1 in row k)
+    if (wv == 0) {
+        real dm = R(0.0);
+        Kahan kdm;
+        auto add = [&](real v) {
+            if (PREC) kdm.add(v);
+            else dm = dm + v;
+        };
+        int k = 0;
+        for (; k + TILE_PAD <= nz; k += TILE_PAD) {
+#pragma unroll
+            for (int q = 0; q < TILE_PAD; ++q) add(Ldv[(k + q) * S]);
+        }
+        for (; k < nz; ++k) add(Ldv[k * S]);
+        Lsum[0] = PREC ? kdm.s : dm;
+    }
+    __syncthreads();
+    const real dmdt_pp = Lsum[0];
+    const real mupp = mupp_old + dtau * ((dmdt_pp + rf) + rmu);
+    const real muts = mut + mupp;
+    const real muave = R(0.5) * (one_p * mupp + one_m * mupp_old);
+#pragma unroll
+    for (int q = 0; q < L; ++q) {
+        const int k = k0 + q;
+        if (k < k1) Ldv[k * S] = dnw[k] * (c1h[k] * (dmdt_pp + rmu) + dv[q]);
+    }
+    __syncthreads();
+    if (wv == 0) {
+        real w = R(0.0);
+        Kahan kww;
+        auto run = [&](int k, real inc) {
+            if (PREC) {
+                kww.add(-inc);
+                w = kww.s;
+            } else {
+                w = w - inc;
+            }
+            Ldv[k * S] = w;
+        };
+        int k = 0;
+        for (; k + TILE_PAD <= nz - 1; k += TILE_PAD) {
+            real v[TILE_PAD];
+#pragma unroll
+            for (int q = 0; q < TILE_PAD; ++q) v[q] = Ldv[(k + q) * S];
+#pragma unroll
+            for (int q = 0; q < TILE_PAD; ++q) run(k + q, v[q]);
+        }
+        for (; k < nz - 1; ++k) run(k, Ldv[k * S]);
+        Ldv[(nz - 1) * S] = R(0.0);
+    }
+    __syncthreads();
+    // the loads of step 3 and the factors' gamma
+    const bool ready = s.gam_ready != 0;
+    auto gam_at = [&](int r) -> tri {
+        if constexpr (PREC) return d.tri64[r * st + c];
+        else return gld(d.gam, 0, r * sm + oc);
+    };
+    const int kb = k0 > 0 ? k0 - 1 : 0;
+    const real th_b = theta(kb, kb * sm + oc);
+    const int kt = k1 < nz ? k1 : nz - 1;
+    const real th_a = theta(kt, kt * sm + oc);
+    const real ph_b = phfull(kb, kb * sm + oc);
+    real ph[L + 1];                              // full phi at w levels k0..
+    ph[0] = phfull(k0, k0 * sm + oc);
+    // Omega'' at w levels k0-1, k0
+    const real ww_b = k0 > 1 ? Ldv[(k0 - 2) * S] : R(0.0);
+    real ww_k = k0 > 0 ? Ldv[(k0 - 1) * S] : R(0.0);
+    auto put_ww = [&](int k, real v) {
+        if (!WW) return;
+        if (s.sum == 0) {
+            gst(d.ww_pp, 0, k * sm + oc, v);
+        } else {
+            const real acc = (s.sum == 1) ? R(0.0) : gld(d.ww_m, 0, k * sm + oc);
+            gst(d.ww_m, 0, k * sm + oc, acc + v);
+        }
+    };
+    auto cfm_at = [&](int k) { return c1f[k] * mut + c2f[k]; };
+
+    // 3. theta'', phi'' right-hand side, rows
+    const real ghalf_eps = (R(0.5) * G_F) * one_m;
+    const real c_force = (R(0.5) * dtau) * G_F;
+    const real c_buoy = dtau * G_F;
+    // right-hand side of row r from D, A of the layers r and r-1
+    auto row = [&](int r, real wo, real rw, real D, real Dm, real A, real Am) {
+        real pg = (c_force * rdn[r]) * (D - Dm);
+        if (XO && s.cq) pg = gld(d.cqw, 0, r * sm + oc) * pg;             // moist_cq
+        const real t1 = dtau * rw + pg;
+        const real t3 = c_buoy * (rdn[r] * (A - Am) - c1f[r] * muave);
+        return wo + (t1 + t3);
+    };
+    auto dph = [&](real r1, real r0, real p1, real p0) {
+        return one_p * (r1 - r0) + one_m * (p1 - p0);
+    };
+    // EOS parts E1, E2 of a level: p'' = c2a (E1 - al''), al'' from E2
+    real rhs[L], c2a[L], E1[L], E2[L];
+    real ph0 = R(0.0);                          // phi'' at the first level
+    real A_0 = R(0.0), D_0 = R(0.0), wo_0 = R(0.0), rw_0 = R(0.0);   // first
+    real A_l = R(0.0), Am_l = R(0.0), B_l = R(0.0), Dm_l = R(0.0);   // last
+    real r_l = R(0.0), p_l = R(0.0), wo_l = R(0.0), rw_l = R(0.0);
+    real c2a_l = R(0.0), t2_l = R(0.0), alt_l = R(0.0);
+    if (k0 == 0) put_ww(0, R(0.0));
+    {
+        real wd_prev = ((R(0.5) * (ww_k + ww_b)) * rdnw[kb]) * (ph[0] - ph_b);
+        const real wd0 = ww_k * (fnm[ka] * th[0] + fnp[ka] * th_b);
+        real wdtn_k = k0 > 0 ? wd0 : R(0.0);
+#pragma unroll
+        for (int q = 0; q < L; ++q) {
+            if (k0 + q >= k1) continue;
+            const int k = k0 + q;
+            const bool has_up = k + 1 < nz;
+            const unsigned o = bc + q * sm;
+            ph[q + 1] = phfull(k + 1, o + sm);
+            const real told = gld(d.th_pp, 0, o);
+            const real rth = gld(d.rth_t, 0, o);
+            const real pr = gld(d.p, 0, o);
+            const real rph = gld(d.rph_t, 0, o);
+            const real alt = gld(d.alt, 0, o);
+            const real pho = gld(d.ph_pp, 0, o);
+            const real wo = gld(d.w_pp, 0, o);
+            const real rw = gld(d.rw_t, 0, o);
+            const real ww_n = Ldv[k * S];
+            const real th_up = (q + 1 < L && k + 1 < k1) ? th[q + 1 < L ? q + 1 : q] : th_a;
+            const int ku = has_up ? k + 1 : k;
+            const real wdt = ww_n * (fnm[ku] * th_up + fnp[ku] * th[q]);
+            const real wdtn_n = has_up ? wdt : R(0.0);
+            const real thn = told + dtau * (rth - (hxy[q]
+                                            + rdnw[k] * (wdtn_n - wdtn_k)));
+            gst(d.th_pp, 0, o, thn);
+            put_ww(k + 1, ww_n);
+            const real chs = c1h[k] * muts + c2h[k];
+            const real cth = chs * th[q];
+            const real t2 = (R(0.5) * (one_p * thn + one_m * told)) / cth;
+            E2[q] = alt * (c1h[k] * mupp);
+            E1[q] = (alt * (thn - (c1h[k] * mupp) * th[q])) / cth;
+            const real wd = ((R(0.5) * (ww_n + ww_k)) * rdnw[k]) * (ph[q + 1] - ph[q]);
+            c2a[q] = GAMMA_F * pr / alt;
+            const real chm = c1h[k] * mut + c2h[k];
+            const real A = (c2a[q] * alt) * t2;
+            const real B = (c2a[q] * rdnw[k]) / chm;
+            real r = dtau * (rph + ghalf_eps * wo);
+            r = r - dtau * (fnm[k] * wd + fnp[k] * wd_prev);
+            rhs[q] = k == 0 ? R(0.0) : pho + r / cfm_at(k);
+            if (q == 0) {
+                ph0 = pho;
+                A_0 = A; wo_0 = wo; rw_0 = rw;
+            } else {
+                // layer k-1 is complete, and its row unless it is the first
+                const real D = B_l * dph(rhs[q], r_l, pho, p_l);
+                if (q == 1) D_0 = D;
+                else Lr[(k - 1) * S].w = (tri)row(k - 1, wo_l, rw_l, D, Dm_l, A_l, Am_l);
+                Dm_l = D;
+            }
+            Am_l = A_l;
+            A_l = A; B_l = B; r_l = rhs[q]; p_l = pho; wo_l = wo; rw_l = rw;
+            c2a_l = c2a[q]; t2_l = t2; alt_l = alt;
+            wd_prev = wd;
+            ww_k = ww_n;
+            wdtn_k = wdtn_n;
+        }
+    }
+    // w level nz (its owner): phi'' right-hand side
+    real rhs_t = R(0.0), pho_t = R(0.0), wold_t = R(0.0);
+    if (top) {
+        const unsigned o = nz * sm + oc;
+        pho_t = gld(d.ph_pp, 0, o);
+        wold_t = gld(d.w_pp, 0, o);
+        const real r = dtau * (gld(d.rph_t, 0, o) + ghalf_eps * wold_t);
+        rhs_t = pho_t + r / cfm_at(nz);
+        if (s.top_lid) rhs_t = R(0.0);
+    }
+    if (some) {
+        Lx[(wv * X_N + X_RLO) * S] = rhs[0];
+        Lx[(wv * X_N + X_PLO) * S] = ph0;
+        Lx[(wv * X_N + X_RHI) * S] = r_l;
+        Lx[(wv * X_N + X_PHI) * S] = p_l;
+        Lx[(wv * X_N + X_A) * S] = A_l;
+        Lx[(wv * X_N + X_B) * S] = B_l;
+        Lx[(wv * X_N + X_C) * S] = c2a_l;
+    }
+    __syncthreads();
+    real D_dn = R(0.0), A_dn = R(0.0), c2a_dn = R(0.0);
+    real rhs_up = rhs_t, pho_up = pho_t;
+    if (some && k0 > 0) {
+        const real* X = Lx + (wv - 1) * X_N * S;
+        D_dn = X[X_B * S] * dph(rhs[0], X[X_RHI * S], ph0, X[X_PHI * S]);
+        A_dn = X[X_A * S];
+        c2a_dn = X[X_C * S];
+    }
+    if (some && k1 < nz) {
+        rhs_up = Lx[((wv + 1) * X_N + X_RLO) * S];
+        pho_up = Lx[((wv + 1) * X_N + X_PLO) * S];
+    }
+    real cof = R(0.5) * dtau * G_F * one_p;
+    cof = cof * cof;
+    if (some) {
+        // the rows next to other waves' layers
+        const real D_l = B_l * dph(rhs_up, r_l, pho_up, p_l);
+        const bool one = k1 - k0 == 1;
+        if (k0 > 0)
+            Lr[k0 * S].w = (tri)row(k0, wo_0, rw_0, one ? D_l : D_0, D_dn, A_0, A_dn);
+        if (!one)
+            Lr[(k1 - 1) * S].w = (tri)row(k1 - 1, wo_l, rw_l, D_l, Dm_l, A_l, Am_l);
+        if (k0 == 0) {
+            // kinematic lower boundary on w'' from the new u''/v''
+            auto lw = [&](const real* f, unsigned colb, int sl) {
+                return (d.cf1 * gld(f, 0, colb) + d.cf2 * gld(f, sl, colb))
+                       + d.cf3 * gld(f, 2 * sl, colb);
+            };
+            real ue = lw(d.u_pp, ou + RB, stu), uw = lw(d.u_pp, ou, stu);
+            real vn = lw(d.v_pp, oc + RB * nx, stv), vs = lw(d.v_pp, oc, stv);
+            const real* RS ht = d.ht;
+            real h = ht[c];
+            const real w0 =
+                (R(0.5) * s.rdy) * ((ht[jp * nx + i] - h) * vn + (h - ht[jm * nx + i]) * vs)
+                + (R(0.5) * s.rdx) * ((ht[j * nx + ip] - h) * ue + (h - ht[j * nx + im]) * uw);
+            gst(d.w_pp, 0, oc, w0);
+            Lr[0].w = (tri)w0;
+        }
+        // LU factors of the wave's rows
+        real cp = c2a_dn;
+        tri gm[L + 1], gm_l = (tri)R(0.0);       // gamma at rows k0-1..
+        gm[0] = (ready && k0 > 1) ? gam_at(k0 - 1) : (tri)R(0.0);
+#pragma unroll
+        for (int q = 0; q < L; ++q)
+            gm[q + 1] = ready ? gam_at(ka + q < nz ? ka + q : nz - 1) : (tri)R(0.0);
+#pragma unroll
+        for (int q = 0; q < L; ++q) {
+            if (k0 + q >= k1) continue;
+            const int r = k0 + q;
+            if (r >= 1) {
+                // moist_cq: the row's coefficient takes cqw(r) first
+                const tri tcof = (XO && s.cq)
+                    ? (tri)gld(d.cqw, 0, r * sm + oc) * (tri)cof : (tri)cof;
+                const real chmc = c1h[r] * mut + c2h[r];
+                const real chmdn = c1h[r - 1] * mut + c2h[r - 1];
+                const tri rdn_r = rdn[r], rdnw_r = rdnw[r], rdnw_m = rdnw[r - 1];
+                tri a_r = (tri)R(0.0);
+                if (r >= 2)
+                    a_r = -tcof * rdn_r * rdnw_m * (tri)cp
+                          / ((tri)chmdn * (tri)cfm_at(r - 1));
+                const tri b = (tri)R(1.0) + tcof * rdn_r
+                                  * (rdnw_r * (tri)c2a[q] / ((tri)chmc * (tri)cfm_at(r))
+                                     + rdnw_m * (tri)cp
+                                           / ((tri)chmdn * (tri)cfm_at(r)));
+                Lr[r * S].a = a_r;
+                if (ready) {
+                    Lr[r * S].b = (tri)R(1.0) / (b - a_r * (r == 1 ? (tri)R(0.0) : gm[q]));
+                    Lr[r * S].g = gm[q + 1];
+                } else {
+                    Lr[r * S].b = b;
+                    Lr[r * S].g = -tcof * rdn_r * rdnw_r * (tri)c2a[q]
+                                 / ((tri)chmc * (tri)cfm_at(r + 1));
+                }
+            }
+            cp = c2a[q];
+            gm_l = gm[q + 1];
+        }
+        if (top) {
+            // row nz from layer nz-1
+            const real chm_b = c1h[nz - 1] * mut + c2h[nz - 1];
+            tri a_top = (tri)R(0.0);
+            real wtop = R(0.0);
+            if (!s.top_lid) {
+                a_top = -(tri)R(2.0) * (tri)cof * (tri)rdnw[nz - 1]
+                        * (tri)rdnw[nz - 1] * (tri)c2a_l
+                        / ((tri)chm_b * (tri)cfm_at(nz - 1));
+                real dph_dn = dph(rhs_t, r_l, pho_t, p_l);
+                real bterm = dtau * G_F * c2a_l * rdnw[nz - 1] * rdnw[nz - 1]
+                              / chm_b * dph_dn;
+                real cterm = dtau * G_F * (R(2.0) * rdnw[nz - 1] * c2a_l * alt_l * t2_l
+                                            + c1f[nz] * muave);
+                wtop = wold_t + ((dtau * gld(d.rw_t, 0, nz * sm + oc) - bterm) - cterm);
+            }
+            const tri b_top = (tri)R(1.0) + (tri)R(2.0) * (tri)cof * (tri)rdnw[nz - 1]
+                                                * (tri)rdnw[nz - 1] * (tri)c2a_l
+                                                / ((tri)chm_b * (tri)cfm_at(nz));
+            Lr[nz * S].w = (tri)wtop;
+            Lr[nz * S].a = a_top;
+            Lr[nz * S].b = ready ? (tri)R(1.0) / (b_top - a_top * gm_l) : b_top;
+            Lr[nz * S].g = (tri)R(0.0);
+        }
+    }
+    __syncthreads();
+
+    // 4. elimination and back substitution by the first group; rows come from
+    // LDS in blocks of SB, the next block's reads in flight under the current
+    if (wv == 0) {
+        constexpr int SB = 4;
+        tri w = Lr[0].w, gp = (tri)R(0.0);
+        Row v[2][SB];
+        auto get = [&](int r, auto h) {
+#pragma unroll
+            for (int q = 0; q < SB; ++q) v[h][q] = Lr[(r + q) * S];
+        };
+        auto fwd = [&](auto rdy) {
+            constexpr bool RDY = decltype(rdy)::value;
+            auto step = [&](int r, const Row& x_) {
+                tri al = x_.b;
+                if (!RDY) {
+                    al = (tri)R(1.0) / (x_.b - x_.a * gp);
+                    gp = x_.g * al;
+                    Lr[r * S].g = gp;
+                }
+                w = (x_.w - x_.a * w) * al;
+                Lr[r * S].w = w;
+            };
+            const std::integral_constant<int, 0> h0{};
+            const std::integral_constant<int, 1> h1{};
+            int r = 1;
+            get(1, h0);
+            for (; r + 2 * SB - 1 <= nz; r += 2 * SB) {
+                get(r + SB, h1);
+#pragma unroll
+                for (int q = 0; q < SB; ++q) step(r + q, v[0][q]);
+                get(r + 2 * SB, h0);
+#pragma unroll
+                for (int q = 0; q < SB; ++q) step(r + SB + q, v[1][q]);
+            }
+            for (; r <= nz; ++r) step(r, Lr[r * S]);
+        };
+        if (ready) fwd(std::true_type{});
+        else fwd(std::false_type{});
+        struct alignas(2 * sizeof(tri)) Half { tri w, g; };
+        Half u[2][SB];
+        auto geth = [&](int k, auto h) {
+#pragma unroll
+            for (int q = 0; q < SB; ++q)
+                u[h][q] = *reinterpret_cast<const Half*>(&Lr[(k - q) * S]);
+        };
+        auto back = [&](int k, const Half& x_) {
+            w = x_.w - x_.g * w;
+            Lr[k * S].w = w;
+        };
+        const std::integral_constant<int, 0> h0{};
+        const std::integral_constant<int, 1> h1{};
+        int k = nz - 1;
+        geth(k, h0);
+        for (; k - 2 * SB + 1 >= 1; k -= 2 * SB) {
+            geth(k - SB, h1);
+#pragma unroll
+            for (int q = 0; q < SB; ++q) back(k - q, u[0][q]);
+            geth(k - 2 * SB, h0);
+#pragma unroll
+            for (int q = 0; q < SB; ++q) back(k - SB - q, u[1][q]);
+        }
+        for (; k >= 1; --k) {
+            const Half z = {Lr[k * S].w, Lr[k * S].g};
+            back(k, z);
+        }
+    }
+    __syncthreads();
+
+    // 5. w'', damper, phi'', p'' of the wave's levels
+    const real c_ph = ((R(0.5) * dtau) * G_F) * one_p;
+    if (wv == 0) d.mu_pp[c] = mupp;
+    if (!some) return;
+    real phn_lo = R(0.0), hbot = R(0.0);
+    if (DAMP) hbot = phfull(nz, nz * sm + oc) / G_F - s.zdamp;
+#pragma unroll
+    for (int q = 0; q <= L; ++q) {
+        const int k = k0 + q;
+        if (k > k1) continue;
+        const unsigned o = bc + q * sm;
+        real phn;
+        if (k == 0) {
+            phn = ph0;
+        } else {
+            real wf = (real)Lr[k * S].w;
+            if (DAMP) {
+                const real hk = ph[q] / G_F;
+                if (hk >= hbot) {
+                    const real wst = gld(d.w, 0, o);
+                    real arg = (R(1.5707963) * (hk - hbot)) / s.zdamp;
+                    real sn = (real)sin((double)arg);
+                    real dw = (s.dampmag * sn) * sn;
+                    wf = (wf - (dw * cfm_at(k)) * wst) / (R(1.0) + dw);
+                }
+            }
+            const real cfs = c1f[k] * muts + c2f[k];
+            const real rk = (q < L && k < k1) ? rhs[q < L ? q : 0] : rhs_up;
+            phn = rk + (c_ph * wf) / cfs;
+            if (k < k1 || top) {
+                gst(d.w_pp, 0, o, wf);
+                gst(d.ph_pp, 0, o, phn);
+                if (!ready && k < nz) {
+                    if constexpr (PREC) d.tri64[k * st + c] = (double)Lr[k * S].g;
+                    else gst(d.gam, 0, o, (real)Lr[k * S].g);
+                }
+            }
+        }
+        if (q > 0) {
+            const int e = q - 1, h = k - 1;
+            const real chm2 = c1h[h] * muts + c2h[h];
+            const real al = -(E2[e] + rdnw[h] * (phn - phn_lo)) / chm2;
+            if (AL) gst(d.al_pp, 0, o - sm, al);
+            gst(pout, 0, o - sm, c2a[e] * (E1[e] - al));
+        }
+        phn_lo = phn;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Small-step finish (reference dycore.cu:1087-1198) + EOS of the new state
 // ---------------------------------------------------------------------------
@@ -2561,10 +3086,70 @@ static inline size_t park_bytes(const Sc& c, int cols_per_block)
     return (size_t)2 * c.park * cols_per_block * sizeof(real);
 }
 
+// The column solve is tiled up to this many columns.  One thread per column
+// (k_column) then leaves most SIMDs with at most one wave, whose two sweeps
+// wait on one level's loads at a time; beyond it k_column has the waves, and
+// the tile's serial steps and its 4 waves a SIMD cost more.  us a launch,
+// k_column -> k_column_tile: 512 columns x 64 levels 109 -> 14, 3072x30
+// 52 -> 15, 30720x50 (moist) 103 -> 41, 25883x45 (terrain, FP64) 141 -> 75,
+// 50000x49 (terrain) 102 -> 86; but 243987x50 (precision form) 320 -> 428 and
+// 1000000x50 1047 -> 1285.
+constexpr int kTileColumns = 96 * 1024;
+constexpr int kTileX = 16, kTileLevels = 4;
+
+// The tile's launch for nz levels: 16 columns keep a workgroup at 4 waves
+// (nz <= 64), four of them a CU at 112-120 VGPRs; 32 columns were slower
+// (250x200x49 2.15 ms a step against 1.98), as were 64 (2.04, 16 waves that
+// wait for one another) and 8 levels a group (2.28, spills).
+struct ColTile {
+    int groups, rows;     // level groups, LDS rows
+    dim3 block;
+    size_t lds;
+};
+
+// false: k_column's domain, or more levels than a workgroup's 512 threads
+static bool column_tile(int cols, int nz, bool prec, ColTile& t)
+{
+    const size_t tri = prec ? sizeof(double) : sizeof(real);
+    constexpr int gpw = 64 / kTileX;
+    t.groups = (nz + kTileLevels - 1) / kTileLevels;
+    const int ng = (t.groups + gpw - 1) / gpw * gpw;       // whole waves
+    t.rows = nz + 1;
+    t.block = dim3(kTileX, ng);
+    t.lds = (size_t)4 * (t.rows + 2 * TILE_PAD) * kTileX * tri
+            + ((size_t)(t.rows + X_N * t.groups + 1) * kTileX + CF_N * t.rows)
+                  * sizeof(real);
+    return cols <= kTileColumns && ng * kTileX <= 512;
+}
+
+template <bool B3, bool DAMP, bool AL, bool WW, bool PREC, bool XO>
+static void launch_column_tile(const Dom& d, const Sc& s0, real* pout,
+                               const ColTile& t, hipStream_t st)
+{
+    Sc s = s0;
+    s.lds_rows = t.rows;
+    s.lds_groups = t.groups;
+    const dim3 g(xcd_grid((unsigned)(d.ny * d.nx + kTileX - 1) / kTileX));
+    hipLaunchKernelGGL((k_column_tile<B3, DAMP, AL, WW, PREC, XO, kTileX,
+                                      kTileLevels>),
+                       g, t.block, t.lds, st, d, s, pout);
+}
+
 template <bool B3, bool DAMP, bool AL, bool WW>
 static void launch_column(const Dom& d, const Sc& s0, real* pout,
                           hipStream_t st)
 {
+    ColTile t;
+    if (column_tile(d.ny * d.nx, d.nz, s0.prec, t)) {
+        if (xo_active(d, s0))
+            with_prec(s0.prec, [&](auto p) {
+                launch_column_tile<B3, DAMP, AL, WW, decltype(p)::value, true>(
+                    d, s0, pout, t, st);
+            });
+        else
+            launch_column_tile<B3, DAMP, AL, WW, false, false>(d, s0, pout, t, st);
+        return;
+    }
     const Sc s = column_sc(s0);
     const size_t lds = park_bytes(s, 256);
     if (s.prec)

@@ -10,7 +10,8 @@ from oracle import dycore_np as O
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [(1, 1, 3), (5, 3, 3), (64, 4, 4), (65, 5, 7), (130, 1, 33),
+SIZES = [(1, 1, 3), (5, 3, 3), (64, 4, 4), (65, 5, 7), (20, 3, 5), (17, 2, 9),
+         (33, 3, 36), (130, 1, 33),
          (63, 9, 50), (200, 67, 17), (257, 60, 65), (3, 70, 130)]
 
 
