@@ -27,7 +27,7 @@ struct Batch {
 // Workgroups one member needs in each batched launch shape.  BK_COLT is
 // the column solve's: col_tile columns per workgroup (64, 128 or 256,
 // chosen per ensemble); the other column launches keep 256.
-enum BatchKind { BK_COLS, BK_ROWS, BK_TFE, BK_FE, BK_COLT, BK_COUNT };
+enum BatchKind { BK_COLS, BK_ROWS, BK_FE, BK_COLT, BK_COUNT };
 int batch_blocks(const Dom& d, int kind, int col_tile);
 
 // The members' views for one launch role, with the per-shape tables.

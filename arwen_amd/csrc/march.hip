@@ -277,8 +277,10 @@ struct PgfWin {
 // advection (reference advection.cu:424-794), large-step PGF
 // (dycore.cu:98-157), constant-K diffusion (diffusion.cu:22-51), and the
 // u''/v'' small-step initialisation (dycore.cu:947-1010).  The periodic
-// duplicate faces are finished by k_tend_faces_edge.  PREC (precision
-// form): the pressure gradient takes p' from the perturbation-form EOS.
+// duplicate faces (u at i = nx, v at j = ny) take the tendency of face 0,
+// whose stencil inputs are theirs, and start from their own u, u0 (v, v0), in
+// the threads of column i = 0 (row j = 0).  PREC (precision form): the
+// pressure gradient takes p' from the perturbation-form EOS.
 template <class SRC, bool B3, bool DIFF, bool PREC, bool HELD = false,
           bool XO = true>
 __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
@@ -292,6 +294,9 @@ __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
     const RowSeg rs = SRC::many ? row_seg_at(nx, ny, g) : row_seg(nx, ny);
     if (!rs.live) return;
     const int i = rs.i, j = rs.j;
+    const Levels lv_g = level_group(nz);
+    const int k0 = lv_g.k0, k1 = lv_g.k1;
+    if (k0 >= k1) return;
     kreal* c1h = kview(d.c1h);
     kreal* c2h = kview(d.c2h);
     kreal* fnm = kview(d.fnm);
@@ -359,13 +364,21 @@ __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
         return gld(d.p, l, cb) - (B3 ? gld(d.pb, l, cb) : kview(d.pb)[k]);
     };
     auto win_init = [&](PgfWin& X, int row, unsigned cb) {
-        real p0 = pp_at(0, row, cb), p1 = pp_at(1, row, cb);
-        real p2 = pp_at(2, row, cb);
-        X.pp_0 = p0;
-        X.pp_p = p1;
-        X.ph_0 = gld(d.php, row, cb);
-        X.gb_0 = B3 ? gld(d.phb, row, cb) : R(0.0);
-        X.dpn_0 = (d.cf1 * p0 + d.cf2 * p1) + d.cf3 * p2;
+        X.ph_0 = gld(d.php, k0 * st + row, cb);
+        X.gb_0 = B3 ? gld(d.phb, k0 * st + row, cb) : R(0.0);
+        if (k0 == 0) {
+            real p0 = pp_at(0, row, cb), p1 = pp_at(1, row, cb);
+            real p2 = pp_at(2, row, cb);
+            X.pp_0 = p0;
+            X.pp_p = p1;
+            X.dpn_0 = (d.cf1 * p0 + d.cf2 * p1) + d.cf3 * p2;
+        } else {
+            X.pp_m = pp_at(k0 - 1, row, cb);
+            X.pp_0 = pp_at(k0, row, cb);
+            const real np = pp_at(k0 + 1 < nz ? k0 + 1 : nz - 1, row, cb);
+            X.pp_p = (k0 + 1 < nz) ? np : R(0.0);
+            X.dpn_0 = fnm[k0] * X.pp_0 + fnp[k0] * X.pp_m;
+        }
     };
     auto win_load = [&](PgfWin& X, int k, int row, unsigned cb, bool top) {
         X.ph_p = gld(d.php, (k + 1) * st + row, cb);
@@ -395,16 +408,26 @@ __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
 
     real uz[5] = {R(0.0), R(0.0), R(0.0), R(0.0), R(0.0)};
     real vz[5] = {R(0.0), R(0.0), R(0.0), R(0.0), R(0.0)};
-    for (int kk = 0; kk < 3 && kk < nz; ++kk) {
-        uz[2 + kk] = gld(d.u, kk * stu + j * pu, cC);
-        vz[2 + kk] = gld(d.v, kk * stv + j * nx, cC);
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+        const int k = k0 + q - 2;
+        if (k < 0 || k >= nz) continue;
+        uz[q] = gld(d.u, k * stu + j * pu, cC);
+        vz[q] = gld(d.v, k * stv + j * nx, cC);
     }
     // the vertical flux through w level k+1 is the next level's flux
     // through its lower face: carried, not recomputed (level 0's lower
-    // face flux is zero)
+    // face flux is zero; a later group forms its first one)
     real fzu = R(0.0), fzv = R(0.0);
+    if (k0 > 0) {
+        const real wA = gld(d.ww, k0 * st + rA, cC);
+        const real wW = gld(d.ww, k0 * st + rA, cW);
+        const real wS = gld(d.ww, k0 * st + rS, cC);
+        fzu = zf(uz[0], uz[1], uz[2], uz[3], R(0.5) * (wW + wA), k0, nz, fnm, fnp);
+        fzv = zf(vz[0], vz[1], vz[2], vz[3], R(0.5) * (wS + wA), k0, nz, fnm, fnp);
+    }
 
-    for (int k = 0; k < nz; ++k) {
+    for (int k = k0; k < k1; ++k) {
         opaque_all();
         const bool top = k + 1 == nz;
         const real c1 = c1h[k], c2 = c2h[k];
@@ -477,6 +500,13 @@ __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
             gst(d.u_pp, lu + j * pu, cC,
                 (c1 * mtf_u + c2) * gld(d.u0, lu + j * pu, cC)
                     - (c1 * msf_u + c2) * x[3]);
+            if (i == 0) {
+                // the duplicate face nx: the same tendency, its own u, u0
+                gst(d.ru_t, lu + j * pu + nx, cC, t);
+                gst(d.u_pp, lu + j * pu + nx, cC,
+                    (c1 * mtf_u + c2) * gld(d.u0, lu + j * pu + nx, cC)
+                        - (c1 * msf_u + c2) * u_b);
+            }
             uz[0] = uz[1]; uz[1] = uz[2]; uz[2] = uz[3]; uz[3] = uz[4];
             const real un = gld(d.u, (k + 3 < nz ? k + 3 : nz - 1) * stu + j * pu, cC);
             uz[4] = (k + 3 < nz) ? un : R(0.0);
@@ -534,6 +564,13 @@ __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
             gst(d.v_pp, lv + j * nx, cC,
                 (c1 * mtf_v + c2) * gld(d.v0, lv + j * nx, cC)
                     - (c1 * msf_v + c2) * y[3]);
+            if (j == 0) {
+                // the duplicate face ny
+                gst(d.rv_t, lv + ny * nx, cC, t);
+                gst(d.v_pp, lv + ny * nx, cC,
+                    (c1 * mtf_v + c2) * gld(d.v0, lv + ny * nx, cC)
+                        - (c1 * msf_v + c2) * v_b);
+            }
             vz[0] = vz[1]; vz[1] = vz[2]; vz[2] = vz[3]; vz[3] = vz[4];
             const real vn = gld(d.v, (k + 3 < nz ? k + 3 : nz - 1) * stv + j * nx, cC);
             vz[4] = (k + 3 < nz) ? vn : R(0.0);
@@ -541,48 +578,6 @@ __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
         win_shift(A, k, rA, cC);
         win_shift(W, k, rA, cW);
         win_shift(S, k, rS, cC);
-    }
-}
-
-// Periodic duplicate faces of the stage tendencies: the face-nx u tendency
-// equals face 0's (same stencil inputs), the face-ny v tendency equals
-// row 0's; u''/v'' init uses the duplicate's own u/u0 (v/v0).  One thread
-// per (k, j) duplicate u face and per (k, i) duplicate v face.
-template <class SRC>
-__global__ __launch_bounds__(256) void k_tend_faces_edge(typename SRC::Arg a)
-{
-    int m, g;
-    if (!SRC::locate(a, m, g)) return;
-    const Dom& d = SRC::dom(a, m);
-    const int nz = d.nz, ny = d.ny, nx = d.nx;
-    const int pu = nx + 1, stu = ny * pu, stv = (ny + 1) * nx;
-    const int t = g * blockDim.x + threadIdx.x;
-    const real* RS mub = d.mub2d;
-    const real* RS mup = d.mup;
-    const real* RS mup0 = d.mup0;
-    if (t < nz * ny) {
-        const int k = t / ny, j = t - k * ny;
-        const int cA = j * nx, cW = j * nx + nx - 1;
-        const real mA = mub[cA] + mup[cA], mW = mub[cW] + mup[cW];
-        const real mtA = mub[cA] + mup0[cA];
-        const real mtf = R(0.5) * (mtA + (mub[cW] + mup0[cW]));
-        const real msf = R(0.5) * (mA + mW);
-        const real c1 = d.c1h[k], c2 = d.c2h[k];
-        const int f0 = k * stu + j * pu, fd = f0 + nx;
-        d.ru_t[fd] = d.ru_t[f0];
-        d.u_pp[fd] = (c1 * mtf + c2) * d.u0[fd] - (c1 * msf + c2) * d.u[fd];
-    } else if (t < nz * ny + nz * nx) {
-        const int r = t - nz * ny;
-        const int k = r / nx, i = r - k * nx;
-        const int cA = i, cS = (ny - 1) * nx + i;
-        const real mA = mub[cA] + mup[cA], mS = mub[cS] + mup[cS];
-        const real mtA = mub[cA] + mup0[cA];
-        const real mtf = R(0.5) * (mtA + (mub[cS] + mup0[cS]));
-        const real msf = R(0.5) * (mA + mS);
-        const real c1 = d.c1h[k], c2 = d.c2h[k];
-        const int f0 = k * stv + i, fd = f0 + ny * nx;
-        d.rv_t[fd] = d.rv_t[f0];
-        d.v_pp[fd] = (c1 * mtf + c2) * d.v0[fd] - (c1 * msf + c2) * d.v[fd];
     }
 }
 
@@ -615,6 +610,9 @@ __global__ __launch_bounds__(256) void k_tend_cols(typename SRC::Arg a, Sc s)
     const RowSeg rs = SRC::many ? row_seg_at(nx, ny, g) : row_seg(nx, ny);
     if (!rs.live) return;
     const int i = rs.i, j = rs.j;
+    const Levels lv_g = level_group(nz);
+    const int k0 = lv_g.k0, k1 = lv_g.k1;
+    if (k0 >= k1) return;
     kreal* c1h = kview(d.c1h);
     kreal* c2h = kview(d.c2h);
     kreal* c1f = kview(d.c1f);
@@ -658,7 +656,7 @@ __global__ __launch_bounds__(256) void k_tend_cols(typename SRC::Arg a, Sc s)
     const real mupc = gld(mup, rA, cC);
     const real mt = gld(mub, rA, cC) + gld(d.mup0, rA, cC);
     const real mupp = gld(d.mup0, rA, cC) - mupc;
-    gst(d.mu_pp, rA, cC, mupp);
+    if (k0 == 0) gst(d.mu_pp, rA, cC, mupp);
     const real qx = s.qrdx, qy = s.qrdy;
 
     auto thb_at = [&](int k, int row, unsigned cb) {
@@ -689,19 +687,24 @@ __global__ __launch_bounds__(256) void k_tend_cols(typename SRC::Arg a, Sc s)
     // windows
     real thz[5] = {R(0.0), R(0.0), R(0.0), R(0.0), R(0.0)};   // theta k-2..k+2
     real wz[5] = {R(0.0), R(0.0), R(0.0), R(0.0), R(0.0)};    // w k-2..k+2
-    for (int kk = 0; kk < 3; ++kk) {
-        if (kk < nz) thz[2 + kk] = th_at(kk, rA, cC);
-        wz[2 + kk] = gld(d.w, kk * st + rA, cC);
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+        const int k = k0 + q - 2;
+        if (k < 0) continue;
+        if (k < nz) thz[q] = th_at(k, rA, cC);
+        if (k <= nz) wz[q] = gld(d.w, k * st + rA, cC);
     }
-    real ww_m = R(0.0), ww_0 = gld(d.ww, rA, cC), ww_p = gld(d.ww, st + rA, cC);
-    real ph_m = R(0.0), ph_0 = phw_at(0, rA, cC), ph_p = phw_at(1, rA, cC);
+    const int l0 = k0 * st;
+    real ww_m = R(0.0), ww_0 = gld(d.ww, l0 + rA, cC), ww_p = gld(d.ww, l0 + st + rA, cC);
+    real ph_m = R(0.0), ph_0 = phw_at(k0, rA, cC), ph_p = phw_at(k0 + 1, rA, cC);
     real pp_m = R(0.0);
     real ru_i_m = R(0.0), ru_ip_m = R(0.0), rv_j_m = R(0.0), rv_jp_m = R(0.0);
     real u_i_m = R(0.0), u_i_mm = R(0.0), u_ip_m = R(0.0), u_ip_mm = R(0.0);
     real v_j_m = R(0.0), v_j_mm = R(0.0), v_jp_m = R(0.0), v_jp_mm = R(0.0);
-    real thp_m = R(0.0), thp_0 = gld(d.thp, rA, cC);
-    real thp_p = gld(d.thp, st + rA, cC);
-    real phpp_0 = gld(d.php0, rA, cC) - gld(d.php, rA, cC);
+    real thp_m = R(0.0), thp_0 = gld(d.thp, l0 + rA, cC);
+    const real thp_1 = gld(d.thp, (k0 + 1 < nz ? l0 + st : l0) + rA, cC);
+    real thp_p = (k0 + 1 < nz) ? thp_1 : R(0.0);
+    real phpp_0 = gld(d.php0, l0 + rA, cC) - gld(d.php, l0 + rA, cC);
     // moist: total water (qv + qc) + qr at the level below (buoyancy)
     real qt_m = R(0.0), qt_mm = R(0.0);
     const real mubc = (MOIST || PREC) ? gld(mub, rA, cC) : R(0.0);
@@ -710,10 +713,55 @@ __global__ __launch_bounds__(256) void k_tend_cols(typename SRC::Arg a, Sc s)
         const real albk = B3 ? gld(d.alb, k * st + rA, cC) : alb1[k];
         return -(dnw[k] * (c1h[k] * mubc + c2h[k])) * albk;
     };
+    auto pp_at = [&](int k, real p_k) {
+        if (PREC) return gld(d.pp, k * st + rA, cC);
+        return p_k - (B3 ? gld(d.pb, k * st + rA, cC) : pb1[k]);
+    };
+    auto qt_at = [&](int lm) {
+        real q = (gld(d.qv, lm + rA, cC) + gld(d.qc, lm + rA, cC))
+                 + gld(d.qr, lm + rA, cC);
+        // a mixed-phase scheme's condensate masses, in order
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (XO && e < d.n_load) q = q + gld(d.qx[e], lm + rA, cC);
+        return q;
+    };
+    // u, v and the coupled fluxes of mass level k on the column's faces
+    auto faces_at = [&](int k, real& ui, real& uip, real& vj, real& vjp,
+                        real& rui, real& ruip, real& rvj, real& rvjp) {
+        const int lu = k * stu, lv = k * stv;
+        ui = gld(d.u, lu + j * pu, cC);
+        const real ui1 = gld(d.u, lu + j * pu, ci1);
+        uip = gld(d.u, lu + j * pu, cx[4]);
+        vj = gld(d.v, lv + rA, cC);
+        const real vj1 = gld(d.v, lv + (j + 1) * nx, cC);
+        vjp = gld(d.v, lv + rN, cC);
+        rui = (c1h[k] * mux_i + c2h[k]) * ui;
+        ruip = (c1h[k] * mux_ip + c2h[k]) * ui1;
+        rvj = (c1h[k] * muy_j + c2h[k]) * vj;
+        rvjp = (c1h[k] * muy_jp + c2h[k]) * vj1;
+    };
 
     // vertical fluxes through the upper face of the level below, carried
     // up the column: theta's at w level k, w's at mass level k-1
     real fzt = R(0.0), fzw = R(0.0);
+    if (k0 > 0) {
+        // a later group starts from the levels below its own
+        const int lb = l0 - st;
+        ww_m = gld(d.ww, lb + rA, cC);
+        ph_m = phw_at(k0 - 1, rA, cC);
+        thp_m = gld(d.thp, lb + rA, cC);
+        pp_m = pp_at(k0 - 1, gld(d.p, lb + rA, cC));
+        if (MOIST) qt_m = qt_at(lb);
+        faces_at(k0 - 1, u_i_m, u_ip_m, v_j_m, v_jp_m, ru_i_m, ru_ip_m, rv_j_m,
+                 rv_jp_m);
+        fzt = zf(thz[0], thz[1], thz[2], thz[3], ww_0, k0, nz, fnm, fnp);
+        const real vel = R(0.5) * (ww_m + ww_0);
+        const real lin = R(0.5) * vel * (wz[2] + wz[1]);
+        real cub = flux3(wz[0], wz[1], wz[2], wz[3], vel);
+        keep(cub);
+        fzw = (k0 == 1) ? lin : cub;
+    }
 
     // kinds: 0 = surface level (w level 0 + mass level 0), 1 = interior,
     // 2 = lid (w level nz only)
@@ -730,33 +778,13 @@ __global__ __launch_bounds__(256) void k_tend_cols(typename SRC::Arg a, Sc s)
         real qt_0 = R(0.0);
         if (mass) {
             p_k = gld(d.p, lm + rA, cC);
-            if (PREC)
-                pp_0 = gld(d.pp, lm + rA, cC);
-            else
-                pp_0 = p_k - (B3 ? gld(d.pb, lm + rA, cC) : pb1[k]);
-            if (MOIST) {
-                qt_0 = (gld(d.qv, lm + rA, cC) + gld(d.qc, lm + rA, cC))
-                       + gld(d.qr, lm + rA, cC);
-                // a mixed-phase scheme's condensate masses, in order
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (XO && e < d.n_load) qt_0 = qt_0 + gld(d.qx[e], lm + rA, cC);
-            }
+            pp_0 = pp_at(k, p_k);
+            if (MOIST) qt_0 = qt_at(lm);
         }
         real ru_i = R(0.0), ru_ip = R(0.0), rv_j = R(0.0), rv_jp = R(0.0);
         real u_i = R(0.0), u_ip = R(0.0), v_j = R(0.0), v_jp = R(0.0);
         if (mass) {
-            const int lu = k * stu, lv = k * stv;
-            u_i = gld(d.u, lu + j * pu, cC);
-            const real u_i1 = gld(d.u, lu + j * pu, ci1);
-            u_ip = gld(d.u, lu + j * pu, cx[4]);
-            v_j = gld(d.v, lv + rA, cC);
-            const real v_j1 = gld(d.v, lv + (j + 1) * nx, cC);
-            v_jp = gld(d.v, lv + rN, cC);
-            ru_i = (c1h[k] * mux_i + c2h[k]) * u_i;
-            ru_ip = (c1h[k] * mux_ip + c2h[k]) * u_i1;
-            rv_j = (c1h[k] * muy_j + c2h[k]) * v_j;
-            rv_jp = (c1h[k] * muy_jp + c2h[k]) * v_j1;
+            faces_at(k, u_i, u_ip, v_j, v_jp, ru_i, ru_ip, rv_j, rv_jp);
         }
 
         // --- rw_t: advection + buoyancy + diffusion ---
@@ -991,9 +1019,10 @@ __global__ __launch_bounds__(256) void k_tend_cols(typename SRC::Arg a, Sc s)
         thp_m = thp_0; thp_0 = thp_p;
         thp_p = (k + 2 < nz) ? thp_n : R(0.0);
     };
-    level(0, Kind<0>{});
-    for (int k = 1; k < nz; ++k) level(k, Kind<1>{});
-    level(nz, Kind<2>{});
+    int k = k0;
+    if (k0 == 0) level(k++, Kind<0>{});
+    for (; k < k1; ++k) level(k, Kind<1>{});
+    if (k1 == nz) level(nz, Kind<2>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -2976,9 +3005,45 @@ static void launch_tend_cols_held(const Dom& d, dim3 g, const Sc& s,
                            dim3(64, 4), 0, st, d, s);
 }
 
+// Level groups of a launch of `blocks` 256-thread workgroups, each group at
+// least `least` levels: enough workgroups that every CU of the 256 holds
+// about `fill` of them.
+static inline unsigned level_groups(unsigned blocks, int nz, int fill,
+                                    int least)
+{
+    const unsigned most = (unsigned)(nz / least > 1 ? nz / least : 1);
+    const unsigned want = (256u * fill + blocks - 1) / (blocks ? blocks : 1);
+    return want < 1 ? 1 : (want > most ? most : want);
+}
+
+// k_tend_faces: 4 workgroups a CU (its reserved LDS admits no more), groups
+// down to 2 levels; each group reloads its windows and forms its first lower
+// flux anew.  us a launch, one march per column -> groups: 512x1x64 122 -> 9,
+// 64x48x30 56 -> 9, 192x160x50 103 -> 36, 250x200x49 terrain 117 -> 62.  8 a
+// CU runs 192x160x50 in 1390 us a step against 1384 and the FP64 181x143x45
+// in 1548 against 1521; 4 levels at least costs 64x48x30 20 us of 377.
+static unsigned tend_faces_groups(unsigned blocks, int nz)
+{
+    return level_groups(blocks, nz, 4, 2);
+}
+
+// k_tend_cols: 16 workgroups a CU with 4 levels at least, and down to 2
+// levels while the CUs hold fewer than 4.  us a launch, one march per column
+// -> groups: 512x1x64 164 -> 12, 64x48x30 71 -> 11, 192x160x50 moist 147 -> 49,
+// 250x200x49 terrain 175 -> 78.  8 a CU runs 501x487x50 (precision form) in
+// 6085 us a step against 6010; 2 levels at 16 a CU costs 192x160x50 15 of
+// 1402, and 4 levels everywhere 64x48x30 20 of 377.
+static unsigned tend_cols_groups(unsigned blocks, int nz)
+{
+    const unsigned few = level_groups(blocks, nz, 4, 2);
+    const unsigned most = level_groups(blocks, nz, 16, 4);
+    return few > most ? few : most;
+}
+
 hipError_t run_tend_faces(const Dom& d, const Sc& s, hipStream_t st)
 {
-    const dim3 g = rowseg_grid(d.nx, d.ny);
+    dim3 g = rowseg_grid(d.nx, d.ny);
+    g.y = tend_faces_groups(g.x, d.nz);
     const bool b3 = d.base3d != 0;
     if (s.held && !s.prec) {
         if (b3 && s.diff) launch_tend_faces_held<true, true>(d, g, s, st);
@@ -2992,15 +3057,13 @@ hipError_t run_tend_faces(const Dom& d, const Sc& s, hipStream_t st)
     } else {
         launch_tend_faces<One, false, false>(d, g, s, b3, st);
     }
-    const int n = d.nz * d.ny + d.nz * d.nx;
-    hipLaunchKernelGGL(k_tend_faces_edge<One>, dim3((n + 255) / 256), dim3(256), 0,
-                       st, d);
     return hipGetLastError();
 }
 
 hipError_t run_tend_cols(const Dom& d, const Sc& s, hipStream_t st)
 {
-    const dim3 g = rowseg_grid(d.nx, d.ny);
+    dim3 g = rowseg_grid(d.nx, d.ny);
+    g.y = tend_cols_groups(g.x, d.nz);
     const bool b3 = d.base3d != 0;
     if (s.held && !s.prec) {
         if (b3 && s.diff) launch_tend_cols_held<true, true>(d, g, s, st);
@@ -3020,17 +3083,6 @@ hipError_t run_tend_cols(const Dom& d, const Sc& s, hipStream_t st)
         else launch_tend_cols<One, false, P>(d, g, s, b3, st);
     });
     return hipGetLastError();
-}
-
-// Level groups of a launch of `blocks` 256-thread workgroups, each group at
-// least `least` levels: enough workgroups that every CU of the 256 holds
-// about `fill` of them.
-static inline unsigned level_groups(unsigned blocks, int nz, int fill,
-                                    int least)
-{
-    const unsigned most = (unsigned)(nz / least > 1 ? nz / least : 1);
-    const unsigned want = (256u * fill + blocks - 1) / (blocks ? blocks : 1);
-    return want < 1 ? 1 : (want > most ? most : want);
 }
 
 // k_uv: groups down to 2 levels, 16 workgroups a CU.  Before the groups and
@@ -3257,7 +3309,6 @@ int batch_blocks(const Dom& d, int kind, int col_tile)
     case BK_COLS: return (d.ny * d.nx + 255) / 256;
     case BK_COLT: return (d.ny * d.nx + col_tile - 1) / col_tile;
     case BK_ROWS: return rows;
-    case BK_TFE: return (d.nz * d.ny + d.nz * d.nx + 255) / 256;
     default: return (d.ny + d.nx + 255) / 256;
     }
 }
@@ -3291,11 +3342,11 @@ hipError_t run_tend_faces_b(const BatchSet& b, const Sc& s, bool b3,
                             hipStream_t st)
 {
     const Batch& r = b.k[BK_ROWS];
+    dim3 g = bgrid(r);
+    g.y = tend_faces_groups(g.x, r.nz);
     with_prec(s.prec, [&](auto p) {
-        launch_tend_faces<Many, decltype(p)::value>(r, bgrid(r), s, b3, st);
+        launch_tend_faces<Many, decltype(p)::value>(r, g, s, b3, st);
     });
-    const Batch& e = b.k[BK_TFE];
-    hipLaunchKernelGGL(k_tend_faces_edge<Many>, bgrid(e), dim3(256), 0, st, e);
     return hipGetLastError();
 }
 
@@ -3303,8 +3354,10 @@ hipError_t run_tend_cols_b(const BatchSet& b, const Sc& s, bool b3,
                            hipStream_t st)
 {
     const Batch& r = b.k[BK_ROWS];
+    dim3 g = bgrid(r);
+    g.y = tend_cols_groups(g.x, r.nz);
     with_prec(s.prec, [&](auto p) {
-        launch_tend_cols<Many, false, decltype(p)::value>(r, bgrid(r), s, b3, st);
+        launch_tend_cols<Many, false, decltype(p)::value>(r, g, s, b3, st);
     });
     return hipGetLastError();
 }
