@@ -65,7 +65,8 @@ struct Sc {
     // held mixing tendencies (d.d6_*) join the stage tendencies as they are
     // stored (arw_step only)
     int held;
-    // k_column_tile: rows its LDS arrays are sized for, level groups
+    // k_column_tile: rows its LDS arrays are sized for, level groups;
+    // k_omega: levels its LDS holds, or 0
     int lds_rows, lds_groups;
 };
 
@@ -301,14 +302,6 @@ __device__ __forceinline__ kreal* kview(const real* p)
 __device__ __forceinline__ int xcd_block()
 {
     const int n = (int)gridDim.x, b = (int)blockIdx.x;
-    return (b % ARW_NXCD) * (n / ARW_NXCD) + b / ARW_NXCD;
-}
-
-// The same numbering over the first n workgroups of a launch whose later
-// workgroups do other work (n a multiple of ARW_NXCD).
-__device__ __forceinline__ int xcd_block_n(int n)
-{
-    const int b = (int)blockIdx.x;
     return (b % ARW_NXCD) * (n / ARW_NXCD) + b / ARW_NXCD;
 }
 

@@ -317,7 +317,9 @@ __global__ void k_eos(Dom d)
     int st = d.ny * d.nx;
     if (c >= st) return;
     real mu = mut_at(d, c);
-    for (int k = 0; k < d.nz; ++k) {
+    const Levels l = level_group(d.nz);
+#pragma unroll 2
+    for (int k = l.k0; k < l.k1; ++k) {
         if (PREC) eos_level_pert(d, k, c, st, mu);
         else eos_level(d, k, c, st, mu);
     }
@@ -360,10 +362,14 @@ __global__ void k_faces(Dom d, real* ru, real* rv)
     if (i < d.nx) rv[iV(k, j, i, d.ny, d.nx)] = rv_at(d, k, j, i);
 }
 
-hipError_t run_eos(const Dom& d, hipStream_t st)
+// k_eos: its levels are independent (a group rereads only the geopotential
+// below its first), so groups go down to 2 levels.
+hipError_t run_eos(const Dom& d, hipStream_t st, bool prec)
 {
-    hipLaunchKernelGGL(k_eos<false>, dim3((d.ny * d.nx + 255) / 256),
-                       dim3(256), 0, st, d);
+    dim3 g((d.ny * d.nx + 255) / 256);
+    g.y = level_groups(g.x, d.nz, 32, 2);
+    if (prec) hipLaunchKernelGGL(k_eos<true>, g, dim3(256), 0, st, d);
+    else hipLaunchKernelGGL(k_eos<false>, g, dim3(256), 0, st, d);
     return hipGetLastError();
 }
 
@@ -2159,9 +2165,8 @@ int32_t ARW_API(calc_p_alpha)(const Dom* d, void* stream)
 {
     int32_t rc = check_domain(d);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_eos<false>, col_grid(*d), dim3(256), 0,
-                       (hipStream_t)stream, *d);
-    return launched("k_eos");
+    hipStream_t st = (hipStream_t)stream;
+    return launched(run_eos(*d, st), "k_eos", -1, st);
 }
 
 int32_t ARW_API(stage_fluxes)(const Dom* d, const arw_params* prm,
@@ -2506,11 +2511,7 @@ static int32_t step_impl(const Dom* d, const arw_params* prm, Ckpt* ck,
             Dom de = dd;
             de.thp = o.thp; de.php = o.php; de.mup = o.mup;
             de.qv = (stage == 0) ? QB[0] : (stage == 1 ? QC[0] : QA[0]);
-            if (prec)
-                hipLaunchKernelGGL(k_eos<true>, col_grid(*d), dim3(256), 0, st, de);
-            else
-                hipLaunchKernelGGL(k_eos<false>, col_grid(*d), dim3(256), 0, st, de);
-            if ((rc = launched(hipGetLastError(), "k_eos", KID_SCALARS, st)))
+            if ((rc = launched(run_eos(de, st, prec), "k_eos", KID_SCALARS, st)))
                 return rc;
         }
     }

@@ -26,8 +26,9 @@ struct Batch {
 
 // Workgroups one member needs in each batched launch shape.  BK_COLT is
 // the column solve's: col_tile columns per workgroup (64, 128 or 256,
-// chosen per ensemble); the other column launches keep 256.
-enum BatchKind { BK_COLS, BK_ROWS, BK_FE, BK_COLT, BK_COUNT };
+// chosen per ensemble); BK_TILE's workgroups take 64 columns in four level
+// groups; the other column launches keep 256.
+enum BatchKind { BK_COLS, BK_ROWS, BK_TILE, BK_COLT, BK_COUNT };
 int batch_blocks(const Dom& d, int kind, int col_tile);
 
 // The members' views for one launch role, with the per-shape tables.
@@ -99,6 +100,36 @@ __device__ __forceinline__ const FinishDst& fin_of(const Batch& b, int m,
     return Many::fin(b, m);
 }
 
+// Level groups.  gridDim.y splits the levels of a column march into equal
+// groups, workgroup blockIdx.y marching levels [k0, k1): at few columns one
+// march per column leaves most SIMDs with a single wave or none, waiting on
+// one level's loads at a time.  A group whose k0 is past the end is empty
+// (its waves return at once).
+struct Levels {
+    int k0, k1;
+};
+
+__device__ __forceinline__ Levels level_group(int nz)
+{
+    const int n = ((int)gridDim.y > 1)
+                      ? (nz + (int)gridDim.y - 1) / (int)gridDim.y : nz;
+    Levels l;
+    l.k0 = (int)blockIdx.y * n;
+    l.k1 = l.k0 + n < nz ? l.k0 + n : nz;
+    return l;
+}
+
+// Level groups of a launch of `blocks` 256-thread workgroups, each group at
+// least `least` levels: enough workgroups that every CU of the 256 holds
+// about `fill` of them.
+static inline unsigned level_groups(unsigned blocks, int nz, int fill,
+                                    int least)
+{
+    const unsigned most = (unsigned)(nz / least > 1 ? nz / least : 1);
+    const unsigned want = (256u * fill + blocks - 1) / (blocks ? blocks : 1);
+    return want < 1 ? 1 : (want > most ? most : want);
+}
+
 // Error reporting and argument checks shared by the library's sources
 // (defined in dycore.hip).
 int32_t lib_fail(int32_t code, const char* msg);
@@ -116,8 +147,9 @@ int32_t lib_check_adj_domain(const Dom* d);
 int32_t lib_check_prec(const arw_params* p, const Dom* d);
 
 hipError_t run_omega(const Dom& d, const Sc& s, int do_eos, hipStream_t st);
-// The plain EOS of the state into d.p, d.al, d.alt (dycore.hip, k_eos).
-hipError_t run_eos(const Dom& d, hipStream_t st);
+// The EOS of the state into d.p, d.al, d.alt (and d.pp in the precision
+// form; dycore.hip, k_eos).
+hipError_t run_eos(const Dom& d, hipStream_t st, bool prec = false);
 // Coupled mass fluxes ru, rv of the state (dycore.hip, k_faces).
 hipError_t run_faces(const Dom& d, real* ru, real* rv, hipStream_t st);
 // The advection adjoints of advect_adj.hip (op 0 scalar, 1 u, 2 v, 3 w),

@@ -83,25 +83,57 @@ __device__ __forceinline__ real pgf_val(
 // ---------------------------------------------------------------------------
 
 
+// Tiles of TX columns by a workgroup (TX, NG) of 256 threads: level group v
+// takes the levels [k0, k1).  Groups of whole waves (TX = 64) keep the level
+// index wave-uniform.  Lanes past the last column (live false) load it
+// again and store nothing.
+struct TileCol {
+    int c, x, wv, k0, k1;
+    bool live, in;       // in: the workgroup has columns
+};
+
+template <int TX>
+__device__ __forceinline__ TileCol tile_col(int tile, int st, int nz)
+{
+    TileCol t;
+    t.x = (int)threadIdx.x;
+    t.wv = TX >= 64 ? __builtin_amdgcn_readfirstlane((int)threadIdx.y)
+                    : (int)threadIdx.y;
+    const int c = tile * TX + t.x;
+    t.in = tile * TX < st;
+    t.live = c < st;
+    t.c = t.live ? c : st - 1;
+    constexpr int NG = 256 / TX;
+    const int per = (nz + NG - 1) / NG;
+    t.k0 = t.wv * per < nz ? t.wv * per : nz;
+    t.k1 = t.k0 + per < nz ? t.k0 + per : nz;
+    return t;
+}
+
 // WRF calc_ww_cp (reference dycore.py:102-131): the column sum of the
 // coupled-flux divergence, then Omega by the upward recurrence.  The sum
 // also serves the acoustic substeps as the reference-momentum mass
 // divergence (acoustic.cu:396-405): dnw*div(C(mu_face) u_t*) is the same
-// float32 expression, so one sum serves both.  Pass 1 parks each level's
-// divergence in ww; pass 2 turns it into Omega.  EOS: the stage-start
-// calc_p_alpha (diagnostics.cu:37-89) when the stage state is new; in the
-// precision form (PREC) its perturbation form, eos_pert, which also keeps
-// p' in d.pp.
-template <class SRC, bool EOS, bool B3, bool PREC, bool XO = true>
+// float32 expression, so one sum serves both.  The level groups form the
+// divergence into LDS; the first group then sums it in level order and runs
+// the recurrence from LDS, storing Omega, while the others go on to the EOS.
+// EOS: the stage-start calc_p_alpha (diagnostics.cu:37-89) when the stage
+// state is new; in the precision form (PREC) its perturbation form, eos_pert,
+// which also keeps p' in d.pp.
+template <class SRC, bool EOS, bool B3, bool PREC, bool XO, int TX>
 __global__ __launch_bounds__(256) void k_omega(typename SRC::Arg a, Sc s)
 {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
     int m, g;
     if (!SRC::locate(a, m, g)) return;
     const Dom& d = SRC::dom(a, m);
     const int nz = d.nz, ny = d.ny, nx = d.nx, st = ny * nx;
     const int stu = ny * (nx + 1), stv = (ny + 1) * nx;
-    const int c = (SRC::many ? g : xcd_block()) * blockDim.x + threadIdx.x;
-    if (c >= st) return;
+    const TileCol tc = tile_col<TX>(SRC::many ? g : xcd_block(), st, nz);
+    if (!tc.in) return;                              // the whole workgroup
+    const int c = tc.c, k0 = tc.k0, k1 = tc.k1;
+    real* const Ld = reinterpret_cast<real*>(lds_raw) + tc.x;
+    const bool lds = s.lds_rows != 0;                // else parked in ww
     const int j = c / nx, i = c - j * nx;
     const int ip = (i + 1 == nx) ? 0 : i + 1, im = (i == 0) ? nx - 1 : i - 1;
     const int jp = (j + 1 == ny) ? 0 : j + 1, jm = (j == 0) ? ny - 1 : j - 1;
@@ -112,16 +144,73 @@ __global__ __launch_bounds__(256) void k_omega(typename SRC::Arg a, Sc s)
     unsigned bc = RB * c, bu = RB * (j * (nx + 1) + i), bu1 = bu + RB;
     unsigned bvn = RB * (c + nx);
     const real ms = d.mub2d[c] + d.mup[c];
-    if (EOS) {
+    const real mw = d.mub2d[j * nx + im] + d.mup[j * nx + im];
+    const real me = d.mub2d[j * nx + ip] + d.mup[j * nx + ip];
+    const real mS = d.mub2d[jm * nx + i] + d.mup[jm * nx + i];
+    const real mN = d.mub2d[jp * nx + i] + d.mup[jp * nx + i];
+    const real muxw = R(0.5) * (ms + mw), muxe = R(0.5) * (me + ms);
+    const real muys = R(0.5) * (ms + mS), muyn = R(0.5) * (mN + ms);
+#pragma unroll 4
+    for (int k = k0; k < k1; ++k) {
+        colb_opaque(bc); colb_opaque(bu); colb_opaque(bu1); colb_opaque(bvn);
+        const real c1 = c1h[k], c2 = c2h[k];
+        real ruw = (c1 * muxw + c2) * gld(d.u, k * stu, bu);
+        real rue = (c1 * muxe + c2) * gld(d.u, k * stu, bu1);
+        real rvs = (c1 * muys + c2) * gld(d.v, k * stv, bc);
+        real rvn = (c1 * muyn + c2) * gld(d.v, k * stv, bvn);
+        const real divv = dnw[k] * (s.rdx * (rue - ruw) + s.rdy * (rvn - rvs));
+        if (lds) Ld[k * TX] = divv;
+        else gst(d.ww, (k + 1) * st, bc, divv);
+    }
+    __syncthreads();
+    if (!tc.live) return;
+    if (tc.wv == 0) {
+        real dmdt = R(0.0), rf = R(0.0);
+        Kahan ksum;
+#pragma unroll 8
+        for (int k = 0; k < nz; ++k) {
+            const real divv = lds ? Ld[k * TX] : gld(d.ww, (k + 1) * st, bc);
+            if (PREC) {
+                ksum.add(divv);
+            } else {
+                dmdt = (k == 0) ? divv : dmdt + divv;
+                rf = rf + divv;
+            }
+        }
+        if (PREC) {
+            // precision form: the compensated column sum serves both
+            dmdt = ksum.s;
+            rf = ksum.s;
+        }
+        gst(d.ww, 0, bc, R(0.0));
+        real run = R(0.0);
+        Kahan krun;
+#pragma unroll 8
+        for (int k = 0; k < nz - 1; ++k) {
+            const real divv = lds ? Ld[k * TX] : gld(d.ww, (k + 1) * st, bc);
+            real inc = (c1h[k] * dnw[k]) * dmdt + divv;
+            if (PREC) {
+                krun.add(inc);
+                run = krun.s;
+            } else {
+                run = run + inc;
+            }
+            gst(d.ww, (k + 1) * st, bc, -run);
+        }
+        gst(d.ww, nz * st, bc, R(0.0));
+        d.dmdt_rf[c] = rf;
+        d.rmu_t[c] = R(0.0);
+    }
+    if (EOS && k0 < k1) {
         kreal* thb1 = kview(d.thb);
         kreal* phb1 = kview(d.phb);
         kreal* alb1 = kview(d.alb);
         kreal* pb1 = kview(d.pb);
         const real mupc = d.mup[c];
-        real ph_lo = gld(d.php, 0, bc);
-        real gb_lo = B3 ? gld(d.phb, 0, bc) : phb1[0];
+        real ph_lo = gld(d.php, k0 * st, bc);
+        real gb_lo = B3 ? gld(d.phb, k0 * st, bc) : phb1[k0];
 #pragma unroll 2
-        for (int k = 0; k < nz; ++k) {
+        for (int k = k0; k < k1; ++k) {
             colb_opaque(bc);
             const unsigned h = k * st;
             const real ph_hi = gld(d.php, h + st, bc);
@@ -154,55 +243,6 @@ __global__ __launch_bounds__(256) void k_omega(typename SRC::Arg a, Sc s)
             gb_lo = gb_hi;
         }
     }
-    const real mw = d.mub2d[j * nx + im] + d.mup[j * nx + im];
-    const real me = d.mub2d[j * nx + ip] + d.mup[j * nx + ip];
-    const real mS = d.mub2d[jm * nx + i] + d.mup[jm * nx + i];
-    const real mN = d.mub2d[jp * nx + i] + d.mup[jp * nx + i];
-    const real muxw = R(0.5) * (ms + mw), muxe = R(0.5) * (me + ms);
-    const real muys = R(0.5) * (ms + mS), muyn = R(0.5) * (mN + ms);
-    real dmdt = R(0.0), rf = R(0.0);
-    Kahan ksum;
-#pragma unroll 4
-    for (int k = 0; k < nz; ++k) {
-        colb_opaque(bc); colb_opaque(bu); colb_opaque(bu1); colb_opaque(bvn);
-        const real c1 = c1h[k], c2 = c2h[k];
-        real ruw = (c1 * muxw + c2) * gld(d.u, k * stu, bu);
-        real rue = (c1 * muxe + c2) * gld(d.u, k * stu, bu1);
-        real rvs = (c1 * muys + c2) * gld(d.v, k * stv, bc);
-        real rvn = (c1 * muyn + c2) * gld(d.v, k * stv, bvn);
-        real divv = dnw[k] * (s.rdx * (rue - ruw) + s.rdy * (rvn - rvs));
-        if (PREC) {
-            ksum.add(divv);
-        } else {
-            dmdt = (k == 0) ? divv : dmdt + divv;
-            rf = rf + divv;
-        }
-        gst(d.ww, (k + 1) * st, bc, divv);
-    }
-    if (PREC) {
-        // precision form: the compensated column sum serves both
-        dmdt = ksum.s;
-        rf = ksum.s;
-    }
-    gst(d.ww, 0, bc, R(0.0));
-    real run = R(0.0);
-    Kahan krun;
-#pragma unroll 4
-    for (int k = 0; k < nz - 1; ++k) {
-        colb_opaque(bc);
-        const unsigned h = (k + 1) * st;
-        real inc = (c1h[k] * dnw[k]) * dmdt + gld(d.ww, h, bc);
-        if (PREC) {
-            krun.add(inc);
-            run = krun.s;
-        } else {
-            run = run + inc;
-        }
-        gst(d.ww, h, bc, -run);
-    }
-    gst(d.ww, nz * st, bc, R(0.0));
-    d.dmdt_rf[c] = rf;
-    d.rmu_t[c] = R(0.0);
 }
 
 // ---------------------------------------------------------------------------
@@ -239,25 +279,6 @@ __device__ __forceinline__ RowSeg row_seg_at(int nx, int ny, int L)
     r.j = __builtin_amdgcn_readfirstlane(by * 4 + (int)threadIdx.y);
     r.live = r.i < nx && r.j < ny;
     return r;
-}
-
-// Level groups.  gridDim.y splits the levels of a column march into equal
-// groups, workgroup blockIdx.y marching levels [k0, k1): at few columns one
-// march per column leaves most SIMDs with a single wave or none, waiting on
-// one level's loads at a time.  A group whose k0 is past the end is empty
-// (its waves return at once).
-struct Levels {
-    int k0, k1;
-};
-
-__device__ __forceinline__ Levels level_group(int nz)
-{
-    const int n = ((int)gridDim.y > 1)
-                      ? (nz + (int)gridDim.y - 1) / (int)gridDim.y : nz;
-    Levels l;
-    l.k0 = (int)blockIdx.y * n;
-    l.k1 = l.k0 + n < nz ? l.k0 + n : nz;
-    return l;
 }
 
 static inline dim3 rowseg_grid(int nx, int ny)
@@ -2267,73 +2288,14 @@ __global__ __launch_bounds__(512) void k_column_tile(Dom d, Sc s, real* RS pout)
 // Small-step finish (reference dycore.cu:1087-1198) + EOS of the new state
 // ---------------------------------------------------------------------------
 
-// Coupled-to-uncoupled fold of one face (reference dycore.cu:1087-1127):
-// new = (C(mu_t*) x_t* + x'') / C(mu_t* + mu'').
-template <int STRIDE_KIND>
-__device__ __forceinline__ void finish_face(const Dom& d, real* RS out,
-                                            const real* RS x,
-                                            const real* RS xpp, int f,
-                                            real msf, real mnf)
-{
-    const int nz = d.nz, ny = d.ny, nx = d.nx;
-    const int sf = STRIDE_KIND == 0 ? ny * (nx + 1) : (ny + 1) * nx;
-    kreal* c1h = kview(d.c1h);
-    kreal* c2h = kview(d.c2h);
-    const unsigned bf = RB * f;
-    // a lone column per thread: unrolled, with no per-level opaque offset,
-    // so several levels' loads are in flight at once
-#pragma unroll 8
-    for (int k = 0; k < nz; ++k) {
-        const real c1 = c1h[k], c2 = c2h[k];
-        gst(out, k * sf, bf, ((c1 * msf + c2) * gld(x, k * sf, bf)
-                              + gld(xpp, k * sf, bf)) / (c1 * mnf + c2));
-    }
-}
-
 struct FinIn {
     real u = R(0.0), upp = R(0.0), v = R(0.0), vpp = R(0.0);
     real w = R(0.0), wpp = R(0.0), php = R(0.0), phpp = R(0.0);
     real thp = R(0.0), thpp = R(0.0);
     real thb = R(0.0), phb = R(0.0), alb = R(0.0);   // terrain base
     real pb = R(0.0);                                // terrain, PREC
+    real u2 = R(0.0), upp2 = R(0.0), v2 = R(0.0), vpp2 = R(0.0);  // duplicates
 };
-
-// Periodic duplicate faces of the finish: u at i = nx (t < ny, row t),
-// v at j = ny (ny <= t < ny + nx, column t - ny).  They read their own
-// face's inputs only, so they run beside the interior columns.
-__device__ __forceinline__ void finish_edges(const Dom& d, const FinishDst& o,
-                                             int t)
-{
-    const int ny = d.ny, nx = d.nx;
-    const real* RS mub = d.mub2d;
-    const real* RS mup = d.mup;
-    const real* RS mu_pp = d.mu_pp;
-    if (t < ny) {
-        const int j = t, cA = j * nx, cB = j * nx + nx - 1;
-        const real msA = mub[cA] + mup[cA], mnA = msA + mu_pp[cA];
-        const real msB = mub[cB] + mup[cB], mnB = msB + mu_pp[cB];
-        finish_face<0>(d, o.u, d.u, d.u_pp, j * (nx + 1) + nx,
-                       R(0.5) * (msA + msB), R(0.5) * (mnA + mnB));
-    } else if (t < ny + nx) {
-        const int i = t - ny, cA = i, cB = (ny - 1) * nx + i;
-        const real msA = mub[cA] + mup[cA], mnA = msA + mu_pp[cA];
-        const real msB = mub[cB] + mup[cB], mnB = msB + mu_pp[cB];
-        finish_face<1>(d, o.v, d.v, d.v_pp, ny * nx + i,
-                       R(0.5) * (msA + msB), R(0.5) * (mnA + mnB));
-    }
-}
-
-// The batched launch's duplicate faces (one domain's run inside k_finish).
-template <class SRC>
-__global__ __launch_bounds__(256) void k_finish_edge(typename SRC::Arg a,
-                                                     FinishDst o_arg)
-{
-    int m, g;
-    if (!SRC::locate(a, m, g)) return;
-    const Dom& d = SRC::dom(a, m);
-    const FinishDst& o = fin_of<SRC>(a, m, o_arg);
-    finish_edges(d, o, g * blockDim.x + threadIdx.x);
-}
 
 // Small-step finish (reference dycore.cu:1087-1198) of the mass column
 // (j, i), its u face (j, i) and v face (j, i), then the EOS of the new
@@ -2344,24 +2306,23 @@ __global__ __launch_bounds__(256) void k_finish_edge(typename SRC::Arg a,
 // d.h_diabatic set): the theta fold removes hdt C(mu_s) h_diabatic, what
 // the substeps integrated from the stage tendency's heating term
 // (reference dycore.cu:1186-1194, module_small_step_em.F:408-426).
-template <class SRC, bool B3, bool EOS, bool PREC, bool XO = true>
+// A tile of columns by level groups (tile_col).  The state may be finished in
+// place, so a group takes php of the level above its own before the barrier
+// behind which the first store comes.  The periodic duplicate faces (u at
+// i = nx, v at j = ny) have the masses of face 0 and ride with its threads.
+template <class SRC, bool B3, bool EOS, bool PREC, bool XO, int TX>
 __global__ __launch_bounds__(256) void k_finish(typename SRC::Arg a,
-                                                FinishDst o_arg, real hdt,
-                                                int nmain)
+                                                FinishDst o_arg, real hdt)
 {
     int m, g;
     if (!SRC::locate(a, m, g)) return;
     const Dom& d = SRC::dom(a, m);
     const FinishDst& o = fin_of<SRC>(a, m, o_arg);
-    if (!SRC::many && (int)blockIdx.x >= nmain) {
-        // the launch's last workgroups: the periodic duplicate faces
-        finish_edges(d, o, ((int)blockIdx.x - nmain) * blockDim.x + threadIdx.x);
-        return;
-    }
     const int nz = d.nz, ny = d.ny, nx = d.nx, st = ny * nx;
     const int stu = ny * (nx + 1), stv = (ny + 1) * nx;
-    const int c = (SRC::many ? g : xcd_block_n(nmain)) * blockDim.x + threadIdx.x;
-    if (c >= st) return;
+    const TileCol tc = tile_col<TX>(SRC::many ? g : xcd_block(), st, nz);
+    if (!tc.in) return;                              // the whole workgroup
+    const int c = tc.c, k0 = tc.k0, k1 = tc.k1;
     const int j = c / nx, i = c - j * nx;
     const int im = (i == 0) ? nx - 1 : i - 1;
     const int jm = (j == 0) ? ny - 1 : j - 1;
@@ -2400,6 +2361,14 @@ __global__ __launch_bounds__(256) void k_finish(typename SRC::Arg a,
         L.phpp = gld(d.ph_pp, k * st, bc);
         L.thp = gld(d.thp, km * st, bc);
         L.thpp = gld(d.th_pp, km * st, bc);
+        if (i == 0) {
+            L.u2 = gld(d.u, km * stu + nx, bu);
+            L.upp2 = gld(d.u_pp, km * stu + nx, bu);
+        }
+        if (j == 0) {
+            L.v2 = gld(d.v, km * stv + st, bc);
+            L.vpp2 = gld(d.v_pp, km * stv + st, bc);
+        }
         if (B3) {
             L.thb = gld(d.thb, km * st, bc);
             L.phb = gld(d.phb, k * st, bc);
@@ -2410,14 +2379,44 @@ __global__ __launch_bounds__(256) void k_finish(typename SRC::Arg a,
     real php_lo = R(0.0), thp_lo = R(0.0), thb_lo = R(0.0), phb_lo = R(0.0);
     real alb_lo = R(0.0), pb_lo = R(0.0);
     FinIn nxt;
-    load(nxt, 0);
-    // kinds: 0 = surface (no EOS below), 1 = interior, 2 = top w level
+    load(nxt, k0);
+    // the new php of w level k1, the group's upper face
+    real php_up = gld(d.php, k1 * st, bc) + gld(d.ph_pp, k1 * st, bc);
+    const real phb_up = B3 ? gld(d.phb, k1 * st, bc) : phb1[k1];
+    keep(php_up);
+    __syncthreads();
+    if (!tc.live || k0 >= k1) return;
+    // EOS of mass level k - 1 below w level k
+    auto eos_below = [&](int k, real php_new, real phb_k) {
+        const unsigned h = (k - 1) * st;
+        if (PREC) {
+            const EosPert e = eos_pert(
+                thp_lo, thb_lo, R(0.0), false, alb_lo, pb_lo, mup_new,
+                c1h[k - 1] * mu_eos + c2h[k - 1], c1h[k - 1], rdnw[k - 1],
+                php_new - php_lo);
+            gst(d.alt, h, bc, e.alt);
+            gst(d.al, h, bc, e.al);
+            gst(d.p, h, bc, e.p);
+            gst(d.pp, h, bc, e.pp);
+        } else {
+            real th = thb_lo + thp_lo;
+            real dph = (phb_k + php_new) - (phb_lo + php_lo);
+            real alt, al;
+            eos_alpha<XO>(d, k - 1, mu_eos, dph, alb_lo, c1h[k - 1],
+                      c2h[k - 1], rdnw[k - 1], alt, al);
+            gst(d.alt, h, bc, alt);
+            gst(d.al, h, bc, al);
+            gst(d.p, h, bc, P0_F * pow_gamma((RD_F * th) / (P0_F * alt)));
+        }
+    };
+    // kinds: 0 = the group's first (no EOS below), 1 = interior, 2 = top w
+    // level of the column
     auto level = [&](int k, auto kind) {
         constexpr int K = decltype(kind)::value;
         colb_opaque(bc);
         colb_opaque(bu);
         const FinIn L = nxt;
-        if (K != 2) load(nxt, k + 1);
+        if (K != 2 && (k + 1 < k1 || k1 == nz)) load(nxt, k + 1);
         const unsigned f = k * st;
         if (K != 2) {
             const real c1 = c1h[k], c2 = c2h[k];
@@ -2425,34 +2424,19 @@ __global__ __launch_bounds__(256) void k_finish(typename SRC::Arg a,
                                       / (c1 * mnf_u + c2));
             gst(o.v, k * stv, bc, ((c1 * msf_v + c2) * L.v + L.vpp)
                                       / (c1 * mnf_v + c2));
+            if (i == 0)
+                gst(o.u, k * stu + nx, bu, ((c1 * msf_u + c2) * L.u2 + L.upp2)
+                                               / (c1 * mnf_u + c2));
+            if (j == 0)
+                gst(o.v, k * stv + st, bc, ((c1 * msf_v + c2) * L.v2 + L.vpp2)
+                                               / (c1 * mnf_v + c2));
         }
         gst(o.w, f, bc, ((c1f[k] * msA + c2f[k]) * L.w + L.wpp)
                             / (c1f[k] * mnA + c2f[k]));
         const real php_new = L.php + L.phpp;
         gst(o.php, f, bc, php_new);
         const real phb_k = B3 ? L.phb : phb1[k];
-        if (EOS && K != 0) {
-            const unsigned h = f - st;
-            if (PREC) {
-                const EosPert e = eos_pert(
-                    thp_lo, thb_lo, R(0.0), false, alb_lo, pb_lo, mup_new,
-                    c1h[k - 1] * mu_eos + c2h[k - 1], c1h[k - 1], rdnw[k - 1],
-                    php_new - php_lo);
-                gst(d.alt, h, bc, e.alt);
-                gst(d.al, h, bc, e.al);
-                gst(d.p, h, bc, e.p);
-                gst(d.pp, h, bc, e.pp);
-            } else {
-                real th = thb_lo + thp_lo;
-                real dph = (phb_k + php_new) - (phb_lo + php_lo);
-                real alt, al;
-                eos_alpha<XO>(d, k - 1, mu_eos, dph, alb_lo, c1h[k - 1],
-                          c2h[k - 1], rdnw[k - 1], alt, al);
-                gst(d.alt, h, bc, alt);
-                gst(d.al, h, bc, al);
-                gst(d.p, h, bc, P0_F * pow_gamma((RD_F * th) / (P0_F * alt)));
-            }
-        }
+        if (EOS && K != 0) eos_below(k, php_new, phb_k);
         if (K != 2) {
             const real thbk = B3 ? L.thb : thb1[k];
             real thn;
@@ -2476,10 +2460,11 @@ __global__ __launch_bounds__(256) void k_finish(typename SRC::Arg a,
         php_lo = php_new;
         phb_lo = phb_k;
     };
-    level(0, Kind<0>{});
-    for (int k = 1; k < nz; ++k) level(k, Kind<1>{});
-    level(nz, Kind<2>{});
-    o.mup[c] = mup_new;
+    level(k0, Kind<0>{});
+    for (int k = k0 + 1; k < k1; ++k) level(k, Kind<1>{});
+    if (k1 == nz) level(nz, Kind<2>{});
+    else if (EOS) eos_below(k1, php_up, phb_up);
+    if (k0 == 0) o.mup[c] = mup_new;
 }
 
 
@@ -2893,23 +2878,60 @@ static void with_xo(bool xo, F&& f)
     else f(std::false_type{});
 }
 
-template <bool PREC, bool XO>
-static void launch_omega(const Dom& d, const Sc& s, int do_eos, hipStream_t st)
+// Columns of a k_omega / k_finish tile: 64 by 4 level groups, or, while that
+// is less than a workgroup a CU, 16 by 16.  us a step with 64 and with 16:
+// 512x1x64 393 and 322, 64x48x30 274 and 238, but 250x200x49 terrain 1360 and
+// 1452, FP64 181x143x45 1412 and 1453 (a wave then spans four groups and its
+// level index, rows and coefficients are no longer scalar).
+// One march per column took 46 and 66 us a launch (Omega, finish) at
+// 512x1x64, 52 and 60 at 250x200x49, 299 and 834 at 1000x1000x50.
+static inline int tile_x(int cols)
 {
-    const bool b3 = d.base3d != 0;
+    return cols <= 64 * 256 ? 16 : 64;
+}
+
+// Calls f with the tile's width as a constant.
+template <class F>
+static void with_tile(int tx, F&& f)
+{
+    if (tx == 16) f(std::integral_constant<int, 16>{});
+    else f(std::integral_constant<int, 64>{});
+}
+
+static inline dim3 tiles(const Dom& d, int tx)
+{
+    return dim3(xcd_grid((unsigned)(d.ny * d.nx + tx - 1) / tx));
+}
+
+template <class SRC, bool PREC, bool XO, int TX>
+static void launch_omega(const typename SRC::Arg& a, dim3 g, int nz, const Sc& s0,
+                         int do_eos, bool b3, hipStream_t st)
+{
+    const dim3 b(TX, 256 / TX);
+    // the divergence of more levels than 64 KB hold is parked in ww
+    size_t l = (size_t)nz * TX * sizeof(real);
+    if (l > 64 * 1024) l = 0;
+    Sc s = s0;
+    s.lds_rows = l ? nz : 0;
     if (do_eos && b3)
-        hipLaunchKernelGGL((k_omega<One, true, true, PREC, XO>), cols(d), dim3(256), 0, st, d, s);
+        hipLaunchKernelGGL((k_omega<SRC, true, true, PREC, XO, TX>), g, b, l, st, a, s);
     else if (do_eos)
-        hipLaunchKernelGGL((k_omega<One, true, false, PREC, XO>), cols(d), dim3(256), 0, st, d, s);
+        hipLaunchKernelGGL((k_omega<SRC, true, false, PREC, XO, TX>), g, b, l, st, a, s);
     else
-        hipLaunchKernelGGL((k_omega<One, false, false, PREC, XO>), cols(d), dim3(256), 0, st, d, s);
+        hipLaunchKernelGGL((k_omega<SRC, false, false, PREC, XO, TX>), g, b, l, st, a, s);
 }
 
 hipError_t run_omega(const Dom& d, const Sc& s, int do_eos, hipStream_t st)
 {
-    if (s.prec) launch_omega<true, true>(d, s, do_eos, st);
-    else if (xo_active(d, s)) launch_omega<false, true>(d, s, do_eos, st);
-    else launch_omega<false, false>(d, s, do_eos, st);
+    const bool b3 = d.base3d != 0;
+    const int tx = tile_x(d.ny * d.nx);
+    with_tile(tx, [&](auto t) {
+        constexpr int TX = decltype(t)::value;
+        const dim3 g = tiles(d, TX);
+        if (s.prec) launch_omega<One, true, true, TX>(d, g, d.nz, s, do_eos, b3, st);
+        else if (xo_active(d, s)) launch_omega<One, false, true, TX>(d, g, d.nz, s, do_eos, b3, st);
+        else launch_omega<One, false, false, TX>(d, g, d.nz, s, do_eos, b3, st);
+    });
     return hipGetLastError();
 }
 
@@ -2966,21 +2988,20 @@ static void launch_tend_cols(const typename SRC::Arg& a, dim3 g, const Sc& s,
         hipLaunchKernelGGL((k_tend_cols<SRC, false, false, MOIST, PREC, false, XO>), g, b, 0, st, a, s);
 }
 
-// g: the whole launch; nmain: its leading column workgroups (one domain:
-// the duplicate-face workgroups follow them; batched: unused)
-template <class SRC, bool PREC, bool XO = true>
+template <class SRC, bool PREC, bool XO, int TX>
 static void launch_finish(const typename SRC::Arg& a, dim3 g,
                           const FinishDst& o, bool b3, bool eos,
-                          hipStream_t st, real hdt = R(0.0), int nmain = 0)
+                          hipStream_t st, real hdt = R(0.0))
 {
+    const dim3 b(TX, 256 / TX);
     if (b3 && eos)
-        hipLaunchKernelGGL((k_finish<SRC, true, true, PREC, XO>), g, dim3(256), 0, st, a, o, hdt, nmain);
+        hipLaunchKernelGGL((k_finish<SRC, true, true, PREC, XO, TX>), g, b, 0, st, a, o, hdt);
     else if (b3)
-        hipLaunchKernelGGL((k_finish<SRC, true, false, PREC, XO>), g, dim3(256), 0, st, a, o, hdt, nmain);
+        hipLaunchKernelGGL((k_finish<SRC, true, false, PREC, XO, TX>), g, b, 0, st, a, o, hdt);
     else if (eos)
-        hipLaunchKernelGGL((k_finish<SRC, false, true, PREC, XO>), g, dim3(256), 0, st, a, o, hdt, nmain);
+        hipLaunchKernelGGL((k_finish<SRC, false, true, PREC, XO, TX>), g, b, 0, st, a, o, hdt);
     else
-        hipLaunchKernelGGL((k_finish<SRC, false, false, PREC, XO>), g, dim3(256), 0, st, a, o, hdt, nmain);
+        hipLaunchKernelGGL((k_finish<SRC, false, false, PREC, XO, TX>), g, b, 0, st, a, o, hdt);
 }
 
 // The held-mixing variants: one domain, plain form (arw_step's held
@@ -3003,17 +3024,6 @@ static void launch_tend_cols_held(const Dom& d, dim3 g, const Sc& s,
     else
         hipLaunchKernelGGL((k_tend_cols<One, B3, DIFF, false, false, true>), g,
                            dim3(64, 4), 0, st, d, s);
-}
-
-// Level groups of a launch of `blocks` 256-thread workgroups, each group at
-// least `least` levels: enough workgroups that every CU of the 256 holds
-// about `fill` of them.
-static inline unsigned level_groups(unsigned blocks, int nz, int fill,
-                                    int least)
-{
-    const unsigned most = (unsigned)(nz / least > 1 ? nz / least : 1);
-    const unsigned want = (256u * fill + blocks - 1) / (blocks ? blocks : 1);
-    return want < 1 ? 1 : (want > most ? most : want);
 }
 
 // k_tend_faces: 4 workgroups a CU (its reserved LDS admits no more), groups
@@ -3243,18 +3253,18 @@ hipError_t run_finish(const Dom& d, const FinishDst& o, bool prec,
     const bool eos = d.qv == nullptr;
     const real hdt = d.h_diabatic ? (real)hdiab_dt : R(0.0);
     const bool xo = prec || d.hypsometric_opt == 2 || d.h_diabatic != nullptr;
-    // the column workgroups, then those of the duplicate faces
-    const int nmain = (int)cols(d).x;
-    const dim3 g(nmain + (d.ny + d.nx + 255) / 256);
-    if (xo) {
-        with_prec(prec, [&](auto p) {
-            launch_finish<One, decltype(p)::value>(d, g, o, d.base3d != 0,
-                                                   eos, st, hdt, nmain);
-        });
-    } else {
-        launch_finish<One, false, false>(d, g, o, d.base3d != 0, eos, st,
-                                         hdt, nmain);
-    }
+    const bool b3 = d.base3d != 0;
+    with_tile(tile_x(d.ny * d.nx), [&](auto t) {
+        constexpr int TX = decltype(t)::value;
+        const dim3 g = tiles(d, TX);
+        if (xo)
+            with_prec(prec, [&](auto p) {
+                launch_finish<One, decltype(p)::value, true, TX>(d, g, o, b3, eos,
+                                                                 st, hdt);
+            });
+        else
+            launch_finish<One, false, false, TX>(d, g, o, b3, eos, st, hdt);
+    });
     return hipGetLastError();
 }
 
@@ -3309,7 +3319,7 @@ int batch_blocks(const Dom& d, int kind, int col_tile)
     case BK_COLS: return (d.ny * d.nx + 255) / 256;
     case BK_COLT: return (d.ny * d.nx + col_tile - 1) / col_tile;
     case BK_ROWS: return rows;
-    default: return (d.ny + d.nx + 255) / 256;
+    default: return (d.ny * d.nx + 63) / 64;
     }
 }
 
@@ -3318,23 +3328,14 @@ static inline dim3 bgrid(const Batch& b)
     return dim3(xcd_grid((unsigned)b.total));
 }
 
-template <bool PREC>
-static void launch_omega_b(const Batch& b, const Sc& s, int do_eos, bool b3,
-                           hipStream_t st)
-{
-    if (do_eos && b3)
-        hipLaunchKernelGGL((k_omega<Many, true, true, PREC>), bgrid(b), dim3(256), 0, st, b, s);
-    else if (do_eos)
-        hipLaunchKernelGGL((k_omega<Many, true, false, PREC>), bgrid(b), dim3(256), 0, st, b, s);
-    else
-        hipLaunchKernelGGL((k_omega<Many, false, false, PREC>), bgrid(b), dim3(256), 0, st, b, s);
-}
-
 hipError_t run_omega_b(const BatchSet& b, const Sc& s, int do_eos, bool b3,
                        hipStream_t st)
 {
-    if (s.prec) launch_omega_b<true>(b.k[BK_COLS], s, do_eos, b3, st);
-    else launch_omega_b<false>(b.k[BK_COLS], s, do_eos, b3, st);
+    const Batch& r = b.k[BK_TILE];
+    with_prec(s.prec, [&](auto p) {
+        launch_omega<Many, decltype(p)::value, true, 64>(r, bgrid(r), r.nz, s,
+                                                         do_eos, b3, st);
+    });
     return hipGetLastError();
 }
 
@@ -3415,13 +3416,12 @@ hipError_t run_column_b(const BatchSet& b, const Sc& s, bool b3, int write_al,
 
 hipError_t run_finish_b(const BatchSet& b, bool b3, bool prec, hipStream_t st)
 {
-    const Batch& r = b.k[BK_COLS];
+    const Batch& r = b.k[BK_TILE];
     const FinishDst none = {};
     with_prec(prec, [&](auto p) {
-        launch_finish<Many, decltype(p)::value>(r, bgrid(r), none, b3, true, st);
+        launch_finish<Many, decltype(p)::value, true, 64>(r, bgrid(r), none, b3,
+                                                          true, st);
     });
-    const Batch& e = b.k[BK_FE];
-    hipLaunchKernelGGL(k_finish_edge<Many>, bgrid(e), dim3(256), 0, st, e, none);
     return hipGetLastError();
 }
 
