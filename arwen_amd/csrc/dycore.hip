@@ -480,30 +480,6 @@ __device__ __forceinline__ real scalar_update(const Dom& d, int k, int c,
     return v;
 }
 
-// Unlimited stage update of one scalar, one thread per point: tend = div
-// of qcur with the averaged fluxes ru_m, rv_m, ww_m; qdst = update from
-// q0.  Used where the domain has too few columns for the column marches.
-__global__ void k_scalar_update(Dom d, const real* __restrict__ qcur,
-                                const real* __restrict__ q0,
-                                real* __restrict__ qdst,
-                                const real* __restrict__ mup0, real dt,
-                                int clamp, real rdx, real rdy,
-                                const real* __restrict__ fixed)
-{
-    const int nz = d.nz, ny = d.ny, nx = d.nx;
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int j = blockIdx.y * blockDim.y + threadIdx.y;
-    int k = blockIdx.z;
-    if (i >= nx || j >= ny || k >= nz) return;
-    Arr3 Q{qcur, ny, nx}, RU{d.ru_m, ny, nx + 1}, RV{d.rv_m, ny + 1, nx},
-        RW{d.ww_m, ny, nx};
-    real tend = R(0.0) + adv_scalar(Q, RU, RV, RW, k, j, i, nz, ny, nx,
-                                   d.rdnw, d.fnm, d.fnp, rdx, rdy);
-    const int x = iM(k, j, i, ny, nx);
-    if (fixed) tend = tend + fixed[x];       // held mixing (moist.py:384-386)
-    qdst[x] = scalar_update(d, k, j * nx + i, q0[x], tend, mup0, dt, clamp);
-}
-
 // The held tendency folded into the time-t scalar ahead of the final
 // stage's limiter, in place: h = q0 + dt h / C(mu_t) (reference moist.py:
 // 293-346 _pd_fold_sources).
@@ -672,7 +648,7 @@ __global__ void k_mup_new(Dom d, real* __restrict__ out)
 }
 
 // One stage of the unlimited transport with explicit checkpointed
-// fluxes and masses: the arithmetic of k_scalar_update.
+// fluxes and masses: the arithmetic of k_scalar_cols.
 __global__ void k_tracer_stage(Dom d, const real* __restrict__ qcur,
                                const real* __restrict__ q0,
                                real* __restrict__ qdst,
@@ -1482,10 +1458,13 @@ int32_t substep(const Dom& d, const Sc& s, real* pout, int write_al,
                     KID_COLUMN, st);
 }
 
-// Below this many columns the column marches leave most SIMDs with less
-// than four waves, and the thread-per-point scalar kernels are faster
-// (both are bit-identical).
-constexpr long kScalarColumnsMin = 512L * 512;
+// Up to this many columns the limiter runs thread per point on stored fluxes
+// (its column marches recompute every flux twice and end in a copy): 40x36x30
+// 315 us a step against 327, 96x100x40 with six species 591 against 606; but
+// 192x160x50 1016 against 988, 400x380x50 with ten species 8062 against 6953.
+// Both are bit-identical.  The unlimited update is a column march always: by
+// level groups 96x100x40 runs 591 us a step, thread per point 631.
+constexpr long kPdColumnsMin = 128L * 128;
 
 // Every scalar's RK stage (reference moist.py:434-698): the unlimited
 // flux form, or the positive-definite limiter on the final stage when
@@ -1520,23 +1499,17 @@ int32_t scalar_stage(const Dom& dd, const arw_params* prm, real* const* cur,
             fx[q] = nullptr;
         }
     }
-    if ((long)dd.ny * dd.nx < kScalarColumnsMin) {
+    if (pd && (long)dd.ny * dd.nx < kPdColumnsMin) {
         // few columns: one thread per point (stored limiter fluxes)
         const dim3 cells((dd.nx + 63) / 64, (dd.ny + 3) / 4, dd.nz);
         for (int q = 0; q < nq; ++q) {
-            if (pd) {
-                hipLaunchKernelGGL(k_pd_fluxes, union_grid(dd, dd.nz + 1),
-                                   dim3(64, 4), 0, st, dd, cur[q], q0[q],
-                                   (real)prm->dx, (real)prm->dy, dt);
-                hipLaunchKernelGGL(k_pd_scale, cells, dim3(64, 4), 0, st, dd,
-                                   q0[q], mup0, rdx, rdy, dt);
-                hipLaunchKernelGGL(k_pd_apply, cells, dim3(64, 4), 0, st, dd,
-                                   q0[q], dst[q], mup0, rdx, rdy, dt);
-            } else {
-                hipLaunchKernelGGL(k_scalar_update, cells, dim3(64, 4), 0, st,
-                                   dd, cur[q], q0[q], dst[q], mup0, dt,
-                                   final ? 1 : 0, rdx, rdy, fx[q]);
-            }
+            hipLaunchKernelGGL(k_pd_fluxes, union_grid(dd, dd.nz + 1),
+                               dim3(64, 4), 0, st, dd, cur[q], q0[q],
+                               (real)prm->dx, (real)prm->dy, dt);
+            hipLaunchKernelGGL(k_pd_scale, cells, dim3(64, 4), 0, st, dd,
+                               q0[q], mup0, rdx, rdy, dt);
+            hipLaunchKernelGGL(k_pd_apply, cells, dim3(64, 4), 0, st, dd,
+                               q0[q], dst[q], mup0, rdx, rdy, dt);
             if ((rc = launched(hipGetLastError(), "scalar stage", KID_SCALARS,
                                st)))
                 return rc;
@@ -2740,7 +2713,7 @@ int32_t ARW_API(tracer_adjoint)(const Dom* d, const arw_params* prm,
 }
 
 // One stage of the unlimited scalar update with explicit fluxes and
-// masses (the arithmetic of k_scalar_update; reference moist.py:385-398):
+// masses (the arithmetic of k_scalar_cols; reference moist.py:385-398):
 // q_new = (C(mu_t) q0 + dt flux_div(q; ru, rv, ww)) / C(mu_new), clamped
 // at zero when clamp.
 int32_t ARW_API(scalar_stage)(const Dom* d, const arw_params* prm,

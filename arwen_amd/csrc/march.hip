@@ -164,12 +164,13 @@ __global__ __launch_bounds__(256) void k_omega(typename SRC::Arg a, Sc s)
     }
     __syncthreads();
     if (!tc.live) return;
-    if (tc.wv == 0) {
+    // column sum and recurrence from the divergence at(k)
+    auto chain = [&](auto at) {
         real dmdt = R(0.0), rf = R(0.0);
         Kahan ksum;
 #pragma unroll 8
         for (int k = 0; k < nz; ++k) {
-            const real divv = lds ? Ld[k * TX] : gld(d.ww, (k + 1) * st, bc);
+            const real divv = at(k);
             if (PREC) {
                 ksum.add(divv);
             } else {
@@ -187,8 +188,7 @@ __global__ __launch_bounds__(256) void k_omega(typename SRC::Arg a, Sc s)
         Kahan krun;
 #pragma unroll 8
         for (int k = 0; k < nz - 1; ++k) {
-            const real divv = lds ? Ld[k * TX] : gld(d.ww, (k + 1) * st, bc);
-            real inc = (c1h[k] * dnw[k]) * dmdt + divv;
+            real inc = (c1h[k] * dnw[k]) * dmdt + at(k);
             if (PREC) {
                 krun.add(inc);
                 run = krun.s;
@@ -200,6 +200,10 @@ __global__ __launch_bounds__(256) void k_omega(typename SRC::Arg a, Sc s)
         gst(d.ww, nz * st, bc, R(0.0));
         d.dmdt_rf[c] = rf;
         d.rmu_t[c] = R(0.0);
+    };
+    if (tc.wv == 0) {
+        if (lds) chain([&](int k) { return Ld[k * TX]; });
+        else chain([&](int k) { return gld(d.ww, (k + 1) * st, bc); });
     }
     if (EOS && k0 < k1) {
         kreal* thb1 = kview(d.thb);
@@ -466,6 +470,7 @@ __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
         const real pbW = B3 ? gld(d.pb, lm + rA, cW) : R(0.0);
         const real pbS = B3 ? gld(d.pb, lm + rS, cC) : R(0.0);
         const int lu = k * stu, lv = k * stv;
+        real tu, tv, u_dup, v_dup;
         // ---- u face ----
         {
             real x[7], y[7];
@@ -521,13 +526,8 @@ __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
             gst(d.u_pp, lu + j * pu, cC,
                 (c1 * mtf_u + c2) * gld(d.u0, lu + j * pu, cC)
                     - (c1 * msf_u + c2) * x[3]);
-            if (i == 0) {
-                // the duplicate face nx: the same tendency, its own u, u0
-                gst(d.ru_t, lu + j * pu + nx, cC, t);
-                gst(d.u_pp, lu + j * pu + nx, cC,
-                    (c1 * mtf_u + c2) * gld(d.u0, lu + j * pu + nx, cC)
-                        - (c1 * msf_u + c2) * u_b);
-            }
+            u_dup = u_b;
+            tu = t;
             uz[0] = uz[1]; uz[1] = uz[2]; uz[2] = uz[3]; uz[3] = uz[4];
             const real un = gld(d.u, (k + 3 < nz ? k + 3 : nz - 1) * stu + j * pu, cC);
             uz[4] = (k + 3 < nz) ? un : R(0.0);
@@ -585,13 +585,8 @@ __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
             gst(d.v_pp, lv + j * nx, cC,
                 (c1 * mtf_v + c2) * gld(d.v0, lv + j * nx, cC)
                     - (c1 * msf_v + c2) * y[3]);
-            if (j == 0) {
-                // the duplicate face ny
-                gst(d.rv_t, lv + ny * nx, cC, t);
-                gst(d.v_pp, lv + ny * nx, cC,
-                    (c1 * mtf_v + c2) * gld(d.v0, lv + ny * nx, cC)
-                        - (c1 * msf_v + c2) * v_b);
-            }
+            v_dup = v_b;
+            tv = t;
             vz[0] = vz[1]; vz[1] = vz[2]; vz[2] = vz[3]; vz[3] = vz[4];
             const real vn = gld(d.v, (k + 3 < nz ? k + 3 : nz - 1) * stv + j * nx, cC);
             vz[4] = (k + 3 < nz) ? vn : R(0.0);
@@ -599,6 +594,20 @@ __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
         win_shift(A, k, rA, cC);
         win_shift(W, k, rA, cW);
         win_shift(S, k, rS, cC);
+        // the duplicate faces nx, ny: the tendency of face 0, their own
+        // u, u0 (last, so that the level above stays one block)
+        if (i == 0) {
+            gst(d.ru_t, lu + j * pu + nx, cC, tu);
+            gst(d.u_pp, lu + j * pu + nx, cC,
+                (c1 * mtf_u + c2) * gld(d.u0, lu + j * pu + nx, cC)
+                    - (c1 * msf_u + c2) * u_dup);
+        }
+        if (j == 0) {
+            gst(d.rv_t, lv + ny * nx, cC, tv);
+            gst(d.v_pp, lv + ny * nx, cC,
+                (c1 * mtf_v + c2) * gld(d.v0, lv + ny * nx, cC)
+                    - (c1 * msf_v + c2) * v_dup);
+        }
     }
 }
 
@@ -744,7 +753,11 @@ __global__ __launch_bounds__(256) void k_tend_cols(typename SRC::Arg a, Sc s)
         // a mixed-phase scheme's condensate masses, in order
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            if (XO && e < d.n_load) q = q + gld(d.qx[e], lm + rA, cC);
+            if (XO) {
+                // past the last one: qr again, not added (no branch)
+                const real x = gld(e < d.n_load ? d.qx[e] : d.qr, lm + rA, cC);
+                q = e < d.n_load ? q + x : q;
+            }
         return q;
     };
     // u, v and the coupled fluxes of mass level k on the column's faces
@@ -973,10 +986,13 @@ __global__ __launch_bounds__(256) void k_tend_cols(typename SRC::Arg a, Sc s)
             const real fz1 = zf(thz[1], thz[2], thz[3], thz[4], ww_p, k + 1, nz, fnm, fnp);
             real t2 = div3(fx1 - fx0, fy1 - fy0, fz1 - fzt, s.rdx, s.rdy, rdnw[k]);
             fzt = fz1;
-            if (XO && MOIST && d.h_diabatic) {
+            if (XO && MOIST) {
                 // the retained microphysics heating, coupled with the
-                // stage's column mass (reference dycore.py:572-592)
-                t2 = t2 + (c1h[k] * mA + c2h[k]) * gld(d.h_diabatic, lm + rA, cC);
+                // stage's column mass (reference dycore.py:572-592); without
+                // it theta', not added (no branch)
+                const real* hd = d.h_diabatic;
+                const real h = gld(hd ? hd : d.thp, lm + rA, cC);
+                t2 = hd ? t2 + (c1h[k] * mA + c2h[k]) * h : t2;
             }
             if (DIFF) {
                 real fc = thp_0;
@@ -2523,6 +2539,9 @@ __global__ __launch_bounds__(256) void k_scalar_cols(Dom d, QGroup g,
     ScalCol q;
     if (!scal_col(d, q)) return;
     const int nz = d.nz, ny = d.ny, nx = d.nx, st = ny * nx;
+    const Levels lv_g = level_group(nz);
+    const int k0 = lv_g.k0, k1 = lv_g.k1;
+    if (k0 >= k1) return;
     const int pu = nx + 1, stu = ny * pu, stv = (ny + 1) * nx;
     kreal* c1h = kview(d.c1h);
     kreal* c2h = kview(d.c2h);
@@ -2541,13 +2560,18 @@ __global__ __launch_bounds__(256) void k_scalar_cols(Dom d, QGroup g,
     real qz[NS][5], fz0[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        qz[s][0] = qz[s][1] = R(0.0);
-        qz[s][2] = gld(g.cur[s], q.rA, cC);
-        qz[s][3] = gld(g.cur[s], st + q.rA, cC);
-        qz[s][4] = gld(g.cur[s], 2 * st + q.rA, cC);
-        fz0[s] = R(0.0);                    // no flux through the surface
+#pragma unroll
+        for (int o = 0; o < 5; ++o) {
+            const int k = k0 + o - 2;
+            qz[s][o] = (k >= 0 && k < nz) ? gld(g.cur[s], k * st + q.rA, cC) : R(0.0);
+        }
+        // no flux through the surface; a later group's first lower flux
+        fz0[s] = R(0.0);
+        if (k0 > 0)
+            fz0[s] = zf(qz[s][0], qz[s][1], qz[s][2], qz[s][3],
+                        gld(d.ww_m, k0 * st + q.rA, cC), k0, nz, fnm, fnp);
     }
-    for (int k = 0; k < nz; ++k) {
+    for (int k = k0; k < k1; ++k) {
         opaque_all();
         const int lm = k * st, lu = k * stu + q.j * pu, lv = k * stv;
         const real ru0 = gld(d.ru_m, lu, cC), ru1 = gld(d.ru_m, lu, q.cu1);
@@ -2708,6 +2732,9 @@ __global__ __launch_bounds__(256) void k_pd_scale_cols(
     ScalCol q;
     if (!scal_col(d, q)) return;
     const int nz = d.nz, ny = d.ny, nx = d.nx, st = ny * nx;
+    const Levels lv_g = level_group(nz);
+    const int k0 = lv_g.k0, k1 = lv_g.k1;
+    if (k0 >= k1) return;
     kreal* c1h = kview(d.c1h);
     kreal* c2h = kview(d.c2h);
     kreal* rdnw = kview(d.rdnw);
@@ -2723,11 +2750,20 @@ __global__ __launch_bounds__(256) void k_pd_scale_cols(
     const PdCol m = pd_col(d, q);
     const real mu0 = d.mub2d[c] + mup0[c];
     // stage scalar window q(k-2..k+2), time-t scalar at k, k+1
-    real w[5] = {R(0.0), R(0.0), gld(cur, q.rA, cC), gld(cur, st + q.rA, cC),
-                 gld(cur, 2 * st + q.rA, cC)};
-    real t0 = gld(q0, q.rA, cC), t1 = gld(q0, st + q.rA, cC);
-    real zb_l = R(0.0), zb_c = R(0.0);      // surface face
-    for (int k = 0; k < nz; ++k) {
+    real w[5];
+#pragma unroll
+    for (int o = 0; o < 5; ++o) {
+        const int k = k0 + o - 2;
+        w[o] = (k >= 0 && k < nz) ? gld(cur, k * st + q.rA, cC) : R(0.0);
+    }
+    real t0 = gld(q0, k0 * st + q.rA, cC);
+    real t1 = k0 + 1 < nz ? gld(q0, (k0 + 1) * st + q.rA, cC) : R(0.0);
+    real zb_l = R(0.0), zb_c = R(0.0);      // the group's lower face
+    if (k0 > 0)
+        pd_zface(d, rdnw, c1h, c2h, fnm, fnp, k0, gld(d.ww_m, k0 * st + q.rA, cC),
+                 m.mA, gld(q0, (k0 - 1) * st + q.rA, cC), t0, w[0], w[1], w[2],
+                 w[3], dt, zb_l, zb_c);
+    for (int k = k0; k < k1; ++k) {
         opaque_all();
         const real c1k = c1h[k], c2k = c2h[k];
         const PdFaces f = pd_faces(d, q, m, cur, q0, k, dx, dy, dt, c1k, c2k,
@@ -2771,6 +2807,9 @@ __global__ __launch_bounds__(256) void k_pd_apply_cols(
     ScalCol q;
     if (!scal_col(d, q)) return;
     const int nz = d.nz, ny = d.ny, nx = d.nx, st = ny * nx;
+    const Levels lv_g = level_group(nz);
+    const int k0 = lv_g.k0, k1 = lv_g.k1;
+    if (k0 >= k1) return;
     kreal* c1h = kview(d.c1h);
     kreal* c2h = kview(d.c2h);
     kreal* rdnw = kview(d.rdnw);
@@ -2786,12 +2825,23 @@ __global__ __launch_bounds__(256) void k_pd_apply_cols(
     const PdCol m = pd_col(d, q);
     const real mu0 = d.mub2d[c] + mup0[c];
     const real mu = d.mub2d[c] + (d.mup[c] + d.mu_pp[c]);
-    real w[5] = {R(0.0), R(0.0), gld(cur, q.rA, cC), gld(cur, st + q.rA, cC),
-                 gld(cur, 2 * st + q.rA, cC)};
-    real t0 = gld(q0, q.rA, cC), t1 = gld(q0, st + q.rA, cC);
-    real zb_l = R(0.0), zb_c = R(0.0);
-    real s_b = R(1.0), s0 = gld(sc, q.rA, cC);   // factors at k-1, k
-    for (int k = 0; k < nz; ++k) {
+    real w[5];
+#pragma unroll
+    for (int o = 0; o < 5; ++o) {
+        const int k = k0 + o - 2;
+        w[o] = (k >= 0 && k < nz) ? gld(cur, k * st + q.rA, cC) : R(0.0);
+    }
+    real t0 = gld(q0, k0 * st + q.rA, cC);
+    real t1 = k0 + 1 < nz ? gld(q0, (k0 + 1) * st + q.rA, cC) : R(0.0);
+    real zb_l = R(0.0), zb_c = R(0.0);      // the group's lower face
+    if (k0 > 0)
+        pd_zface(d, rdnw, c1h, c2h, fnm, fnp, k0, gld(d.ww_m, k0 * st + q.rA, cC),
+                 m.mA, gld(q0, (k0 - 1) * st + q.rA, cC), t0, w[0], w[1], w[2],
+                 w[3], dt, zb_l, zb_c);
+    // factors at k-1, k
+    real s_b = k0 > 0 ? gld(sc, (k0 - 1) * st + q.rA, cC) : R(1.0);
+    real s0 = gld(sc, k0 * st + q.rA, cC);
+    for (int k = k0; k < k1; ++k) {
         opaque_all();
         const int lm = k * st;
         const real c1k = c1h[k], c2k = c2h[k];
@@ -3026,34 +3076,30 @@ static void launch_tend_cols_held(const Dom& d, dim3 g, const Sc& s,
                            dim3(64, 4), 0, st, d, s);
 }
 
-// k_tend_faces: 4 workgroups a CU (its reserved LDS admits no more), groups
-// down to 2 levels; each group reloads its windows and forms its first lower
-// flux anew.  us a launch, one march per column -> groups: 512x1x64 122 -> 9,
-// 64x48x30 56 -> 9, 192x160x50 103 -> 36, 250x200x49 terrain 117 -> 62.  8 a
-// CU runs 192x160x50 in 1390 us a step against 1384 and the FP64 181x143x45
-// in 1548 against 1521; 4 levels at least costs 64x48x30 20 us of 377.
-static unsigned tend_faces_groups(unsigned blocks, int nz)
-{
-    return level_groups(blocks, nz, 4, 2);
-}
-
-// k_tend_cols: 16 workgroups a CU with 4 levels at least, and down to 2
-// levels while the CUs hold fewer than 4.  us a launch, one march per column
-// -> groups: 512x1x64 164 -> 12, 64x48x30 71 -> 11, 192x160x50 moist 147 -> 49,
-// 250x200x49 terrain 175 -> 78.  8 a CU runs 501x487x50 (precision form) in
-// 6085 us a step against 6010; 2 levels at 16 a CU costs 192x160x50 15 of
-// 1402, and 4 levels everywhere 64x48x30 20 of 377.
-static unsigned tend_cols_groups(unsigned blocks, int nz)
+// The stencil marches (k_tend_faces, k_tend_cols, the scalar kernels): a group
+// reloads its windows and forms its first lower fluxes anew, so groups go down
+// to 2 levels only until a CU holds 4 workgroups, and to 8 until it has 32 to
+// run one after the other (shorter tails, and the stencil's levels are still
+// in cache).  us a launch, one march per column -> groups: k_tend_faces
+// 512x1x64 122 -> 9, 192x160x50 103 -> 33, 250x200x49 terrain 117 -> 58;
+// k_tend_cols 164 -> 12, 147 -> 38, 175 -> 67.  us a step without the 8-level
+// groups and with them: 523x516x40 with ten species 12 240 -> 11 962
+// (k_tend_faces) and 13 290 -> 12 376 (the scalars), 1000x1000x50 19 774 ->
+// 19 683 and, for k_tend_cols, 19 850 -> 19 698; 4 levels there cost 501x487x50
+// (precision form) 30 of 5 674.  8 workgroups a CU of 2 levels run 192x160x50
+// in 1390 us against 1384, the FP64 181x143x45 in 1548 against 1521; 4 levels
+// at least cost 64x48x30 20 us of 377.
+static unsigned stencil_groups(unsigned blocks, int nz)
 {
     const unsigned few = level_groups(blocks, nz, 4, 2);
-    const unsigned most = level_groups(blocks, nz, 16, 4);
+    const unsigned most = level_groups(blocks, nz, 32, 8);
     return few > most ? few : most;
 }
 
 hipError_t run_tend_faces(const Dom& d, const Sc& s, hipStream_t st)
 {
     dim3 g = rowseg_grid(d.nx, d.ny);
-    g.y = tend_faces_groups(g.x, d.nz);
+    g.y = stencil_groups(g.x, d.nz);
     const bool b3 = d.base3d != 0;
     if (s.held && !s.prec) {
         if (b3 && s.diff) launch_tend_faces_held<true, true>(d, g, s, st);
@@ -3073,7 +3119,7 @@ hipError_t run_tend_faces(const Dom& d, const Sc& s, hipStream_t st)
 hipError_t run_tend_cols(const Dom& d, const Sc& s, hipStream_t st)
 {
     dim3 g = rowseg_grid(d.nx, d.ny);
-    g.y = tend_cols_groups(g.x, d.nz);
+    g.y = stencil_groups(g.x, d.nz);
     const bool b3 = d.base3d != 0;
     if (s.held && !s.prec) {
         if (b3 && s.diff) launch_tend_cols_held<true, true>(d, g, s, st);
@@ -3272,7 +3318,9 @@ hipError_t run_scalar_cols(const Dom& d, const QGroup& g, const real* mup0,
                            real dt, real rdx, real rdy, int clamp,
                            hipStream_t st)
 {
-    const dim3 grid = rowseg_grid(d.nx, d.ny), blk(64, 4);
+    dim3 grid = rowseg_grid(d.nx, d.ny);
+    grid.y = stencil_groups(grid.x, d.nz);
+    const dim3 blk(64, 4);
     switch (g.n) {
     case 1:
         hipLaunchKernelGGL(k_scalar_cols<1>, grid, blk, 0, st, d, g, mup0, dt,
@@ -3300,7 +3348,9 @@ hipError_t run_pd_cols(const Dom& d, const real* cur, const real* q0,
                        real* out, const real* mup0, real dx, real dy,
                        real dxi, real dyi, real dt, hipStream_t st)
 {
-    const dim3 grid = rowseg_grid(d.nx, d.ny), blk(64, 4);
+    dim3 grid = rowseg_grid(d.nx, d.ny);
+    grid.y = stencil_groups(grid.x, d.nz);
+    const dim3 blk(64, 4);
     hipLaunchKernelGGL(k_pd_scale_cols, grid, blk, 0, st, d, cur, q0, mup0,
                        d.pd_sc, dx, dy, dxi, dyi, dt);
     hipLaunchKernelGGL(k_pd_apply_cols, grid, blk, 0, st, d, cur, q0, mup0,
@@ -3344,7 +3394,7 @@ hipError_t run_tend_faces_b(const BatchSet& b, const Sc& s, bool b3,
 {
     const Batch& r = b.k[BK_ROWS];
     dim3 g = bgrid(r);
-    g.y = tend_faces_groups(g.x, r.nz);
+    g.y = stencil_groups(g.x, r.nz);
     with_prec(s.prec, [&](auto p) {
         launch_tend_faces<Many, decltype(p)::value>(r, g, s, b3, st);
     });
@@ -3356,7 +3406,7 @@ hipError_t run_tend_cols_b(const BatchSet& b, const Sc& s, bool b3,
 {
     const Batch& r = b.k[BK_ROWS];
     dim3 g = bgrid(r);
-    g.y = tend_cols_groups(g.x, r.nz);
+    g.y = stencil_groups(g.x, r.nz);
     with_prec(s.prec, [&](auto p) {
         launch_tend_cols<Many, false, decltype(p)::value>(r, g, s, b3, st);
     });

@@ -1,7 +1,9 @@
 """The step's kernels where their launches change shape: one-column and
 ragged domains, the fewest levels, remainders of the level groups and of
-the 64-column tiles, and duplicate faces that differ from face 0.  One step,
-bit-identical to the float32 oracle."""
+the 16- and 64-column tiles, more levels than a tile's LDS holds, and
+duplicate faces that differ from face 0.  One step, bit-identical to the
+float32 oracle; the FP64 build to the float64 oracle but for its pow, whose
+last bit may differ."""
 import numpy as np
 import pytest
 
@@ -12,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 SIZES = [(1, 1, 3), (5, 3, 3), (64, 4, 4), (65, 5, 7), (20, 3, 5), (17, 2, 9),
          (33, 3, 36), (130, 1, 33),
-         (63, 9, 50), (200, 67, 17), (257, 60, 65), (3, 70, 130)]
+         (63, 9, 50), (200, 67, 17), (257, 60, 65), (3, 70, 130),
+         (17, 9, 128), (131, 127, 9), (2, 3, 1030)]
 
 
 def _noisy(case, seed=5):
@@ -28,7 +31,7 @@ def _noisy(case, seed=5):
 
 def _case(kind, nx, ny, nz):
     from arwen_amd import cases as C
-    if kind == "flat":
+    if kind in ("flat", "precision", "fp64"):
         return _noisy(C.ensemble_member(nx, ny, nz, seed=3))
     if kind == "terrain":
         return _noisy(C.stratified_hill(nx=nx, ny=ny, nz=nz, dx=3000.0,
@@ -59,3 +62,32 @@ def test_step_is_bit_identical_at_the_edges_of_the_launch_shapes(kind, size):
     for n, (err, same) in compare(o, g, names).items():
         assert np.all(np.isfinite(getattr(o, n))), n
         assert same == 1.0, f"{n}: rel {err:.3e}, {same:.6f} identical"
+
+
+@pytest.mark.parametrize("size", [(5, 3, 3), (17, 9, 128), (131, 127, 9)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_precision_form_is_bit_identical_there(size):
+    from arwen_amd import dycore
+    case = _case("precision", *size)
+    case.cfg = case.cfg.with_(precision_form=True)
+    o, g = oracle_and_gpu(case)
+    O.step(o, case.cfg)
+    dycore.step(g, case.cfg)
+    for n, (err, same) in compare(o, g, PROG + DIAG).items():
+        assert same == 1.0, f"{n}: rel {err:.3e}, {same:.6f} identical"
+
+
+@pytest.mark.parametrize("size", [(5, 3, 3), (17, 9, 128), (131, 127, 9)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_fp64_build_agrees_there(size):
+    import torch
+    from arwen_amd import dycore
+    from arwen_amd.state import DomainState
+    case = _case("fp64", *size)
+    o = O.from_case(case, np.float64)
+    g = DomainState.from_host(case, dtype=torch.float64)
+    O.step(o, case.cfg)
+    dycore.step(g, case.cfg)
+    # pow's last bit, 2e-16 of a pressure whose differences the step takes
+    for n, (err, _) in compare(o, g, PROG + DIAG).items():
+        assert err < 1e-9, f"{n}: rel {err:.3e}"
