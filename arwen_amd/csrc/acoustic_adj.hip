@@ -235,30 +235,56 @@ __global__ __launch_bounds__(64) void k_adj_lu(Dom d, Sc s, real* lu)
     lu[LU_A * F + nz * st + c] = an;
 }
 
-// S1 with the stage's factors: the two sweeps only.
-__global__ __launch_bounds__(64) void k_adj_s1_lu(Dom d, Fw f, const real* lu)
+// S1 with the stage's factors: the two sweeps only.  A workgroup (TX, 256/TX)
+// stages the rows of TX columns through LDS, all levels' loads in flight at
+// once; its first TX threads run the two recurrences there (one row's loads at
+// a time took 57 us a launch at 192x160x50, where an HBM round trip per row,
+// not bandwidth, was the bound).  Rows of four values, one LDS read each.
+constexpr int S1_TX = 16;
+
+__global__ __launch_bounds__(256) void k_adj_s1_lu(Dom d, Fw f, const real* lu)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    struct alignas(4 * sizeof(real)) Row { real v, gp, al, a; };
+    extern __shared__ __align__(16) unsigned char s1_lds[];
+    Row* const L = reinterpret_cast<Row*>(s1_lds) + threadIdx.x;
     const int st = d.ny * d.nx, nz = d.nz;
-    if (c >= st) return;
+    const int c0 = (int)xcd_block() * S1_TX + (int)threadIdx.x;
+    const bool on = c0 < st;
+    const int c = on ? c0 : st - 1;
+    const int ty = threadIdx.y, ng = blockDim.y;
     const size_t F = (size_t)(nz + 1) * st;
     const real* __restrict__ LWIN = f.s[W_LPH1];
     real* __restrict__ LW = f.s[W_LW];
-    real vprev = R(0.0);
-    for (int k = 1; k <= nz; ++k) {
-        const real gp = k >= 2 ? lu[LU_GP * F + (k - 1) * st + c] : R(0.0);
-        const real v = LWIN[k * st + c] - gp * vprev;
-        vprev = v;
-        LW[k * st + c] = v;
+    for (int k = 1 + ty; k <= nz; k += ng) {
+        Row r;
+        r.v = LWIN[k * st + c];
+        r.gp = k >= 2 ? lu[LU_GP * F + (k - 1) * st + c] : R(0.0);
+        r.al = lu[LU_AL * F + k * st + c];
+        r.a = lu[LU_A * F + k * st + c];
+        L[k * S1_TX] = r;
     }
-    real carry = R(0.0);
-    for (int k = nz; k >= 1; --k) {
-        const int x = k * st + c;
-        const real v = lu[LU_AL * F + x] * (LW[x] + carry);
-        LW[x] = v;
-        carry = -lu[LU_A * F + x] * v;
+    __syncthreads();
+    if (ty == 0) {
+        real vprev = R(0.0);
+#pragma unroll 4
+        for (int k = 1; k <= nz; ++k) {
+            const Row r = L[k * S1_TX];
+            vprev = r.v - r.gp * vprev;
+            L[k * S1_TX].v = vprev;
+        }
+        real carry = R(0.0);
+#pragma unroll 4
+        for (int k = nz; k >= 1; --k) {
+            const Row r = L[k * S1_TX];
+            const real v = r.al * (r.v + carry);
+            L[k * S1_TX].v = v;
+            carry = -r.a * v;
+        }
+        if (on) f.s[W_L0][c] = LWIN[c] + carry;
     }
-    f.s[W_L0][c] = LWIN[c] + carry;
+    __syncthreads();
+    if (!on) return;
+    for (int k = 1 + ty; k <= nz; k += ng) LW[k * st + c] = L[k * S1_TX].v;
 }
 
 // S1: the transposed Thomas solve of one column.
@@ -1273,8 +1299,13 @@ static int32_t substep_adjoint(const Dom* d, const arw_params* prm,
     const dim3 lev((cols + 255) / 256, nz + 1), colg((cols + 63) / 64);
     hipLaunchKernelGGL(k_adj_p1, lev, dim3(256), 0, st, *d, s, a, fw);
     if ((rc = lib_launched(hipGetLastError(), "k_adj_p1"))) return rc;
-    if (lu)
-        hipLaunchKernelGGL(k_adj_s1_lu, colg, dim3(64), 0, st, *d, fw, lu);
+    // a tile's rows fit the LDS up to 639 levels (FP64: 319); more levels form
+    // the factors anew, the same values
+    const size_t rows = (size_t)(nz + 1) * S1_TX * 4 * sizeof(real);
+    if (lu && rows <= 160 * 1024)
+        hipLaunchKernelGGL(k_adj_s1_lu,
+                           dim3(xcd_grid((unsigned)(cols + S1_TX - 1) / S1_TX)),
+                           dim3(S1_TX, 256 / S1_TX), rows, st, *d, fw, lu);
     else
         hipLaunchKernelGGL(k_adj_s1, colg, dim3(64), 0, st, *d, s, fw);
     if ((rc = lib_launched(hipGetLastError(), "k_adj_s1"))) return rc;

@@ -76,9 +76,14 @@ __device__ __forceinline__ real s3(int o)
 // scalar at mass points (reference advection.cu:384-415)
 struct OpScalar {
     static constexpr bool dupx = true, dupy = true, wlev = false;
-    static __device__ real lam(const Args& a, int k, int j, int i)
+    static constexpr bool foldx = false, foldy = false;
+    static __device__ real raw(const Args& a, int k, int j, int i)
     {
         return a.lam[iM(k, j, i, a.ny, a.nx)];
+    }
+    static __device__ real lam(const Args& a, int k, int j, int i)
+    {
+        return raw(a, k, j, i);
     }
     static __device__ real q(const Args& a, int k, int j, int i)
     {
@@ -105,11 +110,15 @@ struct OpScalar {
 // u at u points, column nx duplicating column 0 (advection.cu:572-611)
 struct OpU {
     static constexpr bool dupx = false, dupy = true, wlev = false;
+    static constexpr bool foldx = true, foldy = false;
+    static __device__ real raw(const Args& a, int k, int j, int i)
+    {
+        return a.lam[iU(k, j, i, a.ny, a.nx)];
+    }
     static __device__ real lam(const Args& a, int k, int j, int i)
     {
-        real l = a.lam[iU(k, j, i, a.ny, a.nx)];
-        if (i == 0) l += a.lam[iU(k, j, a.nx, a.ny, a.nx)];
-        return l;
+        const real l = raw(a, k, j, i), d = raw(a, k, j, i == 0 ? a.nx : i);
+        return i == 0 ? l + d : l;
     }
     static __device__ real q(const Args& a, int k, int j, int i)
     {
@@ -143,11 +152,15 @@ struct OpU {
 // v at v points, row ny duplicating row 0 (advection.cu:754-794)
 struct OpV {
     static constexpr bool dupx = true, dupy = false, wlev = false;
+    static constexpr bool foldx = false, foldy = true;
+    static __device__ real raw(const Args& a, int k, int j, int i)
+    {
+        return a.lam[iV(k, j, i, a.ny, a.nx)];
+    }
     static __device__ real lam(const Args& a, int k, int j, int i)
     {
-        real l = a.lam[iV(k, j, i, a.ny, a.nx)];
-        if (j == 0) l += a.lam[iV(k, a.ny, i, a.ny, a.nx)];
-        return l;
+        const real l = raw(a, k, j, i), d = raw(a, k, j == 0 ? a.ny : j, i);
+        return j == 0 ? l + d : l;
     }
     static __device__ real q(const Args& a, int k, int j, int i)
     {
@@ -181,6 +194,11 @@ struct OpV {
 // (advection.cu:1016-1050)
 struct OpW {
     static constexpr bool dupx = true, dupy = true, wlev = true;
+    static constexpr bool foldx = false, foldy = false;
+    static __device__ real raw(const Args& a, int k, int j, int i)
+    {
+        return lam(a, k, j, i);
+    }
     static __device__ real lam(const Args& a, int k, int j, int i)
     {
         if (k == 0 || k == a.nz) return R(0.0);
@@ -220,18 +238,15 @@ struct OpW {
 // velocities of the six faces c0-2..c0+3 that read cell c0.
 // ---------------------------------------------------------------------------
 
-// c in [-3, n + 3) to [0, n): one correction when n >= 4
-__device__ __forceinline__ int wrapc(int c, int n)
-{
-    if (n >= 4) return c < 0 ? c + n : (c >= n ? c - n : c);
-    return pmod(c, n);
-}
-
 template <class OP>
 struct XLine {
     const Args& a;
     int k, j;
     static constexpr bool dup = OP::dupx;
+    static constexpr bool along = OP::foldx, across = OP::foldy;
+    __device__ real raw(int c) const { return OP::raw(a, k, j, c); }
+    __device__ bool twin() const { return j == 0; }   // row ny folds into it
+    __device__ real raw_twin(int c) const { return OP::raw(a, k, a.ny, c); }
     __device__ int n() const { return a.nx; }
     __device__ real rd() const { return a.rdx; }
     __device__ real lam(int c) const { return OP::lam(a, k, j, c); }
@@ -244,6 +259,10 @@ struct YLine {
     const Args& a;
     int k, i;
     static constexpr bool dup = OP::dupy;
+    static constexpr bool along = OP::foldy, across = OP::foldx;
+    __device__ real raw(int c) const { return OP::raw(a, k, c, i); }
+    __device__ bool twin() const { return i == 0; }   // column nx folds into it
+    __device__ real raw_twin(int c) const { return OP::raw(a, k, c, a.nx); }
     __device__ int n() const { return a.ny; }
     __device__ real rd() const { return a.rdy; }
     __device__ real lam(int c) const { return OP::lam(a, k, c, i); }
@@ -258,20 +277,35 @@ struct YLine {
 struct Win {
     real lw[7];           // output adjoint of cells c0-3 .. c0+3
     real vr[6], vl[6];    // velocity of face c0-2+t seen from right / left
+    int ix[7];            // the cells c0-3 .. c0+3
 };
 
+// All loads are unconditional and the duplicates are selected afterwards: a
+// load under a condition makes the wave wait for the one before it.
 template <class L>
 __device__ __forceinline__ void load_win(const L& l, int c0, Win& w)
 {
     const int n = l.n();
+    wrap7(c0, n, w.ix);
 #pragma unroll
-    for (int p = 0; p < 7; ++p) w.lw[p] = l.lam(wrapc(c0 - 3 + p, n));
+    for (int p = 0; p < 7; ++p) w.lw[p] = l.raw(w.ix[p]);
 #pragma unroll
-    for (int t = 0; t < 6; ++t) {
-        const int f = wrapc(c0 - 2 + t, n);
-        w.vr[t] = l.vel(f);
-        w.vl[t] = (L::dup && f == 0) ? l.vel(n) : w.vr[t];
+    for (int t = 0; t < 6; ++t) w.vr[t] = l.vel(w.ix[t + 1]);
+    real fold = R(0.0), vn = R(0.0);
+    if (L::along) fold = l.raw(n);
+    if (L::dup) vn = l.vel(n);
+    if (L::across && l.twin()) {
+#pragma unroll
+        for (int p = 0; p < 7; ++p) w.lw[p] += l.raw_twin(w.ix[p]);
     }
+    if (L::along) {
+#pragma unroll
+        for (int p = 0; p < 7; ++p)
+            w.lw[p] = w.ix[p] == 0 ? w.lw[p] + fold : w.lw[p];
+    }
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+        w.vl[t] = (L::dup && w.ix[t + 1] == 0) ? vn : w.vr[t];
 }
 
 // dL/dq at the window's cell: face c0-2+t reads it as stencil cell
@@ -292,53 +326,50 @@ __device__ __forceinline__ real win_field(const L& l, const Win& w)
 }
 
 // dL/dvel of a face with velocity v, cell adjoints lr / ll on its sides
-// (0 where the face has no such cell) and stencil q[f-3 .. f+2].
+// (0 where the face has no such cell) and stencil q[f-3 .. f+2], the first
+// six of the cells ix around f.
 template <class L>
-__device__ __forceinline__ real face_dvel(const L& l, int f, real v, real lr,
-                                          real ll)
+__device__ __forceinline__ real face_dvel(const L& l, const int (&ix)[7], real v,
+                                          real lr, real ll)
 {
-    const int n = l.n();
     const real s = sgn(v);
     real acc = R(0.0);
 #pragma unroll
     for (int o = 0; o < 6; ++o)
-        acc += (c5(o) + s5(o) * s) * l.q(wrapc(f + o - 3, n));
+        acc += (c5(o) + s5(o) * s) * l.q(ix[o]);
     return l.rd() * (lr - ll) * acc;
 }
 
 // dup line, face f in [0, n], from the window at c0 = f mod n
 template <class L>
-__device__ __forceinline__ real win_dvel_dup(const L& l, int f, int c0,
-                                             const Win& w)
+__device__ __forceinline__ real win_dvel_dup(const L& l, int f, const Win& w)
 {
     const int n = l.n();
     const real v = (f < n) ? w.vr[2] : w.vl[2];
     const real lr = (f < n) ? w.lw[3] : R(0.0);
     const real ll = (f > 0) ? w.lw[2] : R(0.0);
-    return face_dvel(l, c0, v, lr, ll);
+    return face_dvel(l, w.ix, v, lr, ll);
 }
 
-// dup line, face f in [0, n], without a window (a neighbouring line)
+// dup line, face f in [0, n], on a neighbouring line: its window's cells ix
 template <class L>
-__device__ __forceinline__ real dvel_dup(const L& l, int f)
+__device__ __forceinline__ real dvel_dup(const L& l, int f, const int (&ix)[7])
 {
-    const int n = l.n();
-    const real lr = (f < n) ? l.lam(f) : R(0.0);
-    const real ll = (f > 0) ? l.lam(f - 1) : R(0.0);
-    return face_dvel(l, f == n ? 0 : f, l.vel(f), lr, ll);
+    const real a = l.lam(ix[3]), b = l.lam(ix[2]);
+    const real lr = (f < l.n()) ? a : R(0.0);
+    const real ll = (f > 0) ? b : R(0.0);
+    return face_dvel(l, ix, l.vel(f), lr, ll);
 }
 
 // periodic line: dL/dvel of faces c0 and c0+1 from the window at c0, with
 // one shared stencil q[c0-3 .. c0+3]
 template <class L>
-__device__ __forceinline__ void win_dvel_pair(const L& l, int c0,
-                                              const Win& w, real& d0,
+__device__ __forceinline__ void win_dvel_pair(const L& l, const Win& w, real& d0,
                                               real& d1)
 {
-    const int n = l.n();
     real qw[7];
 #pragma unroll
-    for (int p = 0; p < 7; ++p) qw[p] = l.q(wrapc(c0 - 3 + p, n));
+    for (int p = 0; p < 7; ++p) qw[p] = l.q(w.ix[p]);
     const real s0 = sgn(w.vr[2]), s1 = sgn(w.vr[3]);
     real a0 = R(0.0), a1 = R(0.0);
 #pragma unroll
@@ -461,14 +492,14 @@ __global__ void k_adj_scalar(Args a)
         Win w;
         load_win(l, ic, w);
         if (i < nx) gq += win_field(l, w);
-        if (a.gru) a.gru[iU(k, j, i, ny, nx)] += win_dvel_dup(l, i, ic, w);
+        if (a.gru) a.gru[iU(k, j, i, ny, nx)] += win_dvel_dup(l, i, w);
     }
     if (k < nz && i < nx) {
         YLine<OpScalar> l{a, k, i};
         Win w;
         load_win(l, jc, w);
         if (j < ny) gq += win_field(l, w);
-        if (a.grv) a.grv[iV(k, j, i, ny, nx)] += win_dvel_dup(l, j, jc, w);
+        if (a.grv) a.grv[iV(k, j, i, ny, nx)] += win_dvel_dup(l, j, w);
     }
     if (i < nx && j < ny) {
         if (a.gq && k < nz)
@@ -496,7 +527,7 @@ __global__ void k_adj_u(Args a)
         if (i < nx) gq += win_field(l, w);
         if (a.gru) {           // ru[i] enters mass centres i-1 and i
             real d0, d1;
-            win_dvel_pair(l, ic, w, d0, d1);
+            win_dvel_pair(l, w, d0, d1);
             a.gru[iU(k, j, i, ny, nx)] +=
                 R(0.5) * ((i < nx ? d1 : R(0.0)) + (i >= 1 ? d0 : R(0.0)));
         }
@@ -508,8 +539,8 @@ __global__ void k_adj_u(Args a)
         if (j < ny) gq += win_field(l, w);
         if (a.grv)             // rv[., i] enters the y faces of u columns i, i+1
             a.grv[iV(k, j, i, ny, nx)] +=
-                R(0.5) * (win_dvel_dup(l, j, jc, w)
-                          + dvel_dup(YLine<OpU>{a, k, ip}, j));
+                R(0.5) * (win_dvel_dup(l, j, w)
+                          + dvel_dup(YLine<OpU>{a, k, ip}, j, w.ix));
     }
     if (i < nx && j < ny) {
         if (a.gq && k < nz)
@@ -538,8 +569,8 @@ __global__ void k_adj_v(Args a)
         if (i < nx) gq += win_field(l, w);
         if (a.gru)             // ru[j, .] enters the x faces of v rows j, j+1
             a.gru[iU(k, j, i, ny, nx)] +=
-                R(0.5) * (win_dvel_dup(l, i, ic, w)
-                          + dvel_dup(XLine<OpV>{a, k, jp}, i));
+                R(0.5) * (win_dvel_dup(l, i, w)
+                          + dvel_dup(XLine<OpV>{a, k, jp}, i, w.ix));
     }
     if (k < nz && i < nx) {
         YLine<OpV> l{a, k, i};
@@ -548,7 +579,7 @@ __global__ void k_adj_v(Args a)
         if (j < ny) gq += win_field(l, w);
         if (a.grv) {           // rv[j] enters mass centres j-1 and j
             real d0, d1;
-            win_dvel_pair(l, jc, w, d0, d1);
+            win_dvel_pair(l, w, d0, d1);
             a.grv[iV(k, j, i, ny, nx)] +=
                 R(0.5) * ((j < ny ? d1 : R(0.0)) + (j >= 1 ? d0 : R(0.0)));
         }
@@ -577,29 +608,31 @@ __global__ void k_adj_w(Args a)
     real gq = R(0.0);
     if (j < ny && k < nz) {
         real g = R(0.0);
+        Win w;
+        wrap7(ic, nx, w.ix);
         if (own) {
             XLine<OpW> l{a, k, j};
-            Win w;
             load_win(l, ic, w);
             if (i < nx) gq += win_field(l, w);
-            g = a.fnm[k] * win_dvel_dup(l, i, ic, w);
+            g = a.fnm[k] * win_dvel_dup(l, i, w);
         }
         if (a.gru) {           // ru[k] enters levels k (fnm) and k+1 (fnp)
-            if (up) g += a.fnp[k + 1] * dvel_dup(XLine<OpW>{a, k + 1, j}, i);
+            if (up) g += a.fnp[k + 1] * dvel_dup(XLine<OpW>{a, k + 1, j}, i, w.ix);
             a.gru[iU(k, j, i, ny, nx)] += g;
         }
     }
     if (i < nx && k < nz) {
         real g = R(0.0);
+        Win w;
+        wrap7(jc, ny, w.ix);
         if (own) {
             YLine<OpW> l{a, k, i};
-            Win w;
             load_win(l, jc, w);
             if (j < ny) gq += win_field(l, w);
-            g = a.fnm[k] * win_dvel_dup(l, j, jc, w);
+            g = a.fnm[k] * win_dvel_dup(l, j, w);
         }
         if (a.grv) {
-            if (up) g += a.fnp[k + 1] * dvel_dup(YLine<OpW>{a, k + 1, i}, j);
+            if (up) g += a.fnp[k + 1] * dvel_dup(YLine<OpW>{a, k + 1, i}, j, w.ix);
             a.grv[iV(k, j, i, ny, nx)] += g;
         }
     }

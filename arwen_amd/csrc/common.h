@@ -118,6 +118,23 @@ __device__ __forceinline__ int pmod(int i, int n)
     return r < 0 ? r + n : r;
 }
 
+// The periodic cells c0-3 .. c0+3 of a line of n cells, 0 <= c0 < n: one
+// correction each when n >= 4 (the modulo of a variable costs about 30
+// instructions, and a branch a cell would split the loads).
+__device__ __forceinline__ void wrap7(int c0, int n, int (&ix)[7])
+{
+    if (n >= 4) {
+#pragma unroll
+        for (int o = 0; o < 7; ++o) {
+            const int c = c0 + o - 3;
+            ix[o] = c < 0 ? c + n : (c >= n ? c - n : c);
+        }
+    } else {
+#pragma unroll
+        for (int o = 0; o < 7; ++o) ix[o] = pmod(c0 + o - 3, n);
+    }
+}
+
 // Flat indices.  Mass/w fields: (k, j, i) with row width nx; u: nx+1;
 // v: ny+1 rows.  Extents are checked on the host to fit in int32.
 __device__ __forceinline__ int iM(int k, int j, int i, int ny, int nx)

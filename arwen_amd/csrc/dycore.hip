@@ -101,10 +101,13 @@ __device__ real adv_scalar(Q q, RU ru, RV rv, RW rw, int k, int j, int i,
                             real rdx, real rdy)
 {
     real x[7], y[7];
+    int ix[7], iy[7];
+    wrap7(i, nx, ix);
+    wrap7(j, ny, iy);
 #pragma unroll
     for (int o = 0; o < 7; ++o) {
-        x[o] = q(k, j, pmod(i + o - 3, nx));
-        y[o] = q(k, pmod(j + o - 3, ny), i);
+        x[o] = q(k, j, ix[o]);
+        y[o] = q(k, iy[o], i);
     }
     real fx0 = flux5(x[0], x[1], x[2], x[3], x[4], x[5], ru(k, j, i));
     real fx1 = flux5(x[1], x[2], x[3], x[4], x[5], x[6], ru(k, j, i + 1));
@@ -129,15 +132,18 @@ __device__ real adv_u(U u, RU ru, RV rv, RW rw, int k, int j, int i,
     int im = (ic == 0) ? nx - 1 : ic - 1;
     // x faces at mass centres im (left) and ic (right)
     real x[7];
+    int ix[7], iy[7];
+    wrap7(ic, nx, ix);
+    wrap7(j, ny, iy);
 #pragma unroll
-    for (int o = 0; o < 7; ++o) x[o] = u(k, j, pmod(ic + o - 3, nx));
+    for (int o = 0; o < 7; ++o) x[o] = u(k, j, ix[o]);
     real vl = R(0.5) * (ru(k, j, im) + ru(k, j, im + 1));
     real vr = R(0.5) * (ru(k, j, ic) + ru(k, j, ic + 1));
     real fx0 = flux5(x[0], x[1], x[2], x[3], x[4], x[5], vl);
     real fx1 = flux5(x[1], x[2], x[3], x[4], x[5], x[6], vr);
     real y[7];
 #pragma unroll
-    for (int o = 0; o < 7; ++o) y[o] = u(k, pmod(j + o - 3, ny), ic);
+    for (int o = 0; o < 7; ++o) y[o] = u(k, iy[o], ic);
     real v0 = R(0.5) * (rv(k, j, im) + rv(k, j, ic));
     real v1 = R(0.5) * (rv(k, j + 1, im) + rv(k, j + 1, ic));
     real fy0 = flux5(y[0], y[1], y[2], y[3], y[4], y[5], v0);
@@ -162,15 +168,18 @@ __device__ real adv_v(V v, RU ru, RV rv, RW rw, int k, int j, int i,
     int jc = (j >= ny) ? j - ny : j;
     int jm = (jc == 0) ? ny - 1 : jc - 1;
     real x[7];
+    int ix[7], iy[7];
+    wrap7(i, nx, ix);
+    wrap7(jc, ny, iy);
 #pragma unroll
-    for (int o = 0; o < 7; ++o) x[o] = v(k, jc, pmod(i + o - 3, nx));
+    for (int o = 0; o < 7; ++o) x[o] = v(k, jc, ix[o]);
     real u0 = R(0.5) * (ru(k, jm, i) + ru(k, jc, i));
     real u1 = R(0.5) * (ru(k, jm, i + 1) + ru(k, jc, i + 1));
     real fx0 = flux5(x[0], x[1], x[2], x[3], x[4], x[5], u0);
     real fx1 = flux5(x[1], x[2], x[3], x[4], x[5], x[6], u1);
     real y[7];
 #pragma unroll
-    for (int o = 0; o < 7; ++o) y[o] = v(k, pmod(jc + o - 3, ny), i);
+    for (int o = 0; o < 7; ++o) y[o] = v(k, iy[o], i);
     real vl = R(0.5) * (rv(k, jm, i) + rv(k, jm + 1, i));
     real vr = R(0.5) * (rv(k, jc, i) + rv(k, jc + 1, i));
     real fy0 = flux5(y[0], y[1], y[2], y[3], y[4], y[5], vl);
@@ -193,10 +202,13 @@ __device__ real adv_w(W w, RU ru, RV rv, RW rw, int k, int j, int i,
                        const real* __restrict__ fnp, real rdx, real rdy)
 {
     real x[7], y[7];
+    int ix[7], iy[7];
+    wrap7(i, nx, ix);
+    wrap7(j, ny, iy);
 #pragma unroll
     for (int o = 0; o < 7; ++o) {
-        x[o] = w(k, j, pmod(i + o - 3, nx));
-        y[o] = w(k, pmod(j + o - 3, ny), i);
+        x[o] = w(k, j, ix[o]);
+        y[o] = w(k, iy[o], i);
     }
     real u0 = fnm[k] * ru(k, j, i) + fnp[k] * ru(k - 1, j, i);
     real u1 = fnm[k] * ru(k, j, i + 1) + fnp[k] * ru(k - 1, j, i + 1);
@@ -529,8 +541,10 @@ __global__ void k_pd_fluxes(Dom d, const real* __restrict__ qcur,
         const real cr = ((vel * dt) / dx) / muf;
         const real fl = (muf * (dx / dt)) * flux_upwind(q0a(k, j, b), q0a(k, j, a), cr);
         real x[6];
+        int ix[7];
+        wrap7(a, nx, ix);
 #pragma unroll
-        for (int o = 0; o < 6; ++o) x[o] = qc(k, j, pmod(i + o - 3, nx));
+        for (int o = 0; o < 6; ++o) x[o] = qc(k, j, ix[o]);
         const real fh = flux5(x[0], x[1], x[2], x[3], x[4], x[5], vel);
         d.pd_fxl[iU(k, j, i, ny, nx)] = fl;
         d.pd_fxc[iU(k, j, i, ny, nx)] = fh - fl;
@@ -542,8 +556,10 @@ __global__ void k_pd_fluxes(Dom d, const real* __restrict__ qcur,
         const real cr = ((vel * dt) / dy) / muf;
         const real fl = (muf * (dy / dt)) * flux_upwind(q0a(k, b, i), q0a(k, a, i), cr);
         real y[6];
+        int iy[7];
+        wrap7(a, ny, iy);
 #pragma unroll
-        for (int o = 0; o < 6; ++o) y[o] = qc(k, pmod(j + o - 3, ny), i);
+        for (int o = 0; o < 6; ++o) y[o] = qc(k, iy[o], i);
         const real fh = flux5(y[0], y[1], y[2], y[3], y[4], y[5], vel);
         d.pd_fyl[iV(k, j, i, ny, nx)] = fl;
         d.pd_fyc[iV(k, j, i, ny, nx)] = fh - fl;
@@ -806,14 +822,18 @@ __global__ void k_tracer_adj_div(Dom d, const real* __restrict__ m,
     int k = blockIdx.z;
     if (i >= nx || j >= ny || k >= nz) return;
     auto M = [&](int kk, int jj, int ii) { return m[iM(kk, jj, ii, ny, nx)]; };
+    int ix[7], iy[7];
+    wrap7(i, nx, ix);
+    wrap7(j, ny, iy);
     real acc = R(0.0);
+#pragma unroll
     for (int o = 0; o < 6; ++o) {
         // x face f reads cell f + o - 3 == i
-        const int f = pmod(i + 3 - o, nx);
-        const real lx = rdx * (M(k, j, f) - M(k, j, pmod(f - 1, nx)));
+        const int f = ix[6 - o];
+        const real lx = rdx * (M(k, j, f) - M(k, j, f == 0 ? nx - 1 : f - 1));
         acc += w5(o, ru[iU(k, j, f, ny, nx)]) * lx;
-        const int g = pmod(j + 3 - o, ny);
-        const real ly = rdy * (M(k, g, i) - M(k, pmod(g - 1, ny), i));
+        const int g = iy[6 - o];
+        const real ly = rdy * (M(k, g, i) - M(k, g == 0 ? ny - 1 : g - 1, i));
         acc += w5(o, rv[iV(k, g, i, ny, nx)]) * ly;
     }
     // eta faces kf = 1..nz-1 touching cell k
@@ -1044,9 +1064,11 @@ __global__ void k_pda_faces(Dom d, PdWork w, const real* __restrict__ q,
         const real fu = flux_upwind(qb, qa, cr);
         real dqb, dqa, dcr;
         upwind_adj(qb, qa, cr, muf * (dx / dt) * G, dqb, dqa, dcr);
+        int ix[7];
+        wrap7(f >= nx ? f - nx : f, nx, ix);
         real x[6];
 #pragma unroll
-        for (int o = 0; o < 6; ++o) x[o] = cellv(q, k, j, pmod(f + o - 3, nx));
+        for (int o = 0; o < 6; ++o) x[o] = cellv(q, k, j, ix[o]);
         gru[xf] += d5(x, vel) * gc + dcr * (dt / dx) / muf;
         w.hx[xf] = gc;
         w.bx[xf] = dqb;
@@ -1075,9 +1097,11 @@ __global__ void k_pda_faces(Dom d, PdWork w, const real* __restrict__ q,
         const real fu = flux_upwind(qb, qa, cr);
         real dqb, dqa, dcr;
         upwind_adj(qb, qa, cr, muf * (dy / dt) * G, dqb, dqa, dcr);
+        int iy[7];
+        wrap7(g >= ny ? g - ny : g, ny, iy);
         real x[6];
 #pragma unroll
-        for (int o = 0; o < 6; ++o) x[o] = cellv(q, k, pmod(g + o - 3, ny), i);
+        for (int o = 0; o < 6; ++o) x[o] = cellv(q, k, iy[o], i);
         grv[yf] += d5(x, vel) * gc + dcr * (dt / dy) / muf;
         w.hy[yf] = gc;
         w.by[yf] = dqb;
@@ -1138,14 +1162,18 @@ __global__ void k_pda_gather(Dom d, PdWork w, const real* __restrict__ ru,
     if (i >= nx || j >= ny || k >= nz) return;
     const size_t n = (size_t)nz * st;
     const int z0 = iM(k, j, i, ny, nx);
+    int ix[7], iy[7];
+    wrap7(i, nx, ix);
+    wrap7(j, ny, iy);
     real acc = R(0.0);
+#pragma unroll
     for (int o = 0; o < 6; ++o) {
         // x face f reads cell f + o - 3 == i; face nx copies face 0's stencil
-        const int f = pmod(i + 3 - o, nx);
+        const int f = ix[6 - o];
         acc += w5(o, ru[iU(k, j, f, ny, nx)]) * w.hx[iU(k, j, f, ny, nx)];
         if (f == 0)
             acc += w5(o, ru[iU(k, j, nx, ny, nx)]) * w.hx[iU(k, j, nx, ny, nx)];
-        const int g = pmod(j + 3 - o, ny);
+        const int g = iy[6 - o];
         acc += w5(o, rv[iV(k, g, i, ny, nx)]) * w.hy[iV(k, g, i, ny, nx)];
         if (g == 0)
             acc += w5(o, rv[iV(k, ny, i, ny, nx)]) * w.hy[iV(k, ny, i, ny, nx)];
@@ -1748,12 +1776,15 @@ __global__ void k_diff6_rows(Dom d, real coef, int mono, int slope,
     const int ic = (i == nx) ? 0 : i, jc = (j == ny) ? 0 : j;
     const real ten = R(10.0), five = R(5.0), zero = R(0.0), one = R(1.0);
     const real q = R(0.25), h = R(0.5);
+    int ix[7], iy[7];
+    wrap7(ic, nx, ix);
+    wrap7(jc, ny, iy);
     real m[3][3];
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
         for (int b = 0; b < 3; ++b) {
-            const int c = pmod(jc + a - 1, ny) * nx + pmod(ic + b - 1, nx);
+            const int c = iy[a + 2] * nx + ix[b + 2];
             m[a][b] = d.mub2d[c] + d.mup[c];
         }
     // geopotential taps (jc + a - 2, ic + b - 2), a, b in 0..3
@@ -1763,8 +1794,8 @@ __global__ void k_diff6_rows(Dom d, real coef, int mono, int slope,
     for (int a = 0; a < 4; ++a)
 #pragma unroll
         for (int b = 0; b < 4; ++b)
-            ph[a][b] = tap ? d.phb[((size_t)k * ny + pmod(jc + a - 2, ny)) * nx
-                                   + pmod(ic + b - 2, nx)]
+            ph[a][b] = tap ? d.phb[((size_t)k * ny + iy[a + 1]) * nx
+                                   + ix[b + 1]]
                            : zero;
 #define MU(dj, di) m[(dj) + 1][(di) + 1]
 #define PHB(dj, di) ph[(dj) + 2][(di) + 2]
@@ -1772,10 +1803,10 @@ __global__ void k_diff6_rows(Dom d, real coef, int mono, int slope,
                    real cc1, real cc2, real mx0, real mx1, real my0, real my1,
                    real sx0, real sx1, real sy0, real sy1) {
         auto FX = [&](int mm) {
-            return f[((size_t)k * nys + jc) * nxs + pmod(ic + mm, nx)];
+            return f[((size_t)k * nys + jc) * nxs + ix[mm + 3]];
         };
         auto FY = [&](int mm) {
-            return f[((size_t)k * nys + pmod(jc + mm, ny)) * nxs + ic];
+            return f[((size_t)k * nys + iy[mm + 3]) * nxs + ic];
         };
         real px0 = ten * (FX(0) - FX(-1)) - five * (FX(1) - FX(-2)) + (FX(2) - FX(-3));
         real px1 = ten * (FX(1) - FX(0)) - five * (FX(2) - FX(-1)) + (FX(3) - FX(-2));
@@ -1873,24 +1904,28 @@ __global__ void k_diff6q(Dom d, D6Q q, real coef, int mono, int slope,
     const int k = blockIdx.z;
     if (i >= nx || j >= ny || k >= d.nz) return;
     const size_t o = ((size_t)k * ny + j) * nx + i;
-    auto MU = [&](int jj, int ii) {
-        const int c = pmod(jj, ny) * nx + pmod(ii, nx);
+    int ix[7], iy[7];
+    wrap7(i, nx, ix);
+    wrap7(j, ny, iy);
+    // of the column (j + dj, i + di)
+    auto MU = [&](int dj, int di) {
+        const int c = iy[dj + 3] * nx + ix[di + 3];
         return d.mub2d[c] + d.mup[c];
     };
-    auto PHB = [&](int jj, int ii) {
-        return d.phb[((size_t)k * ny + pmod(jj, ny)) * nx + pmod(ii, nx)];
+    auto PHB = [&](int dj, int di) {
+        return d.phb[((size_t)k * ny + iy[dj + 3]) * nx + ix[di + 3]];
     };
     const real ten = R(10.0), five = R(5.0), zero = R(0.0), one = R(1.0);
-    const real mx0 = R(0.5) * (MU(j, i - 1) + MU(j, i));
-    const real mx1 = R(0.5) * (MU(j, i) + MU(j, i + 1));
-    const real my0 = R(0.5) * (MU(j - 1, i) + MU(j, i));
-    const real my1 = R(0.5) * (MU(j, i) + MU(j + 1, i));
+    const real mx0 = R(0.5) * (MU(0, -1) + MU(0, 0));
+    const real mx1 = R(0.5) * (MU(0, 0) + MU(0, 1));
+    const real my0 = R(0.5) * (MU(-1, 0) + MU(0, 0));
+    const real my1 = R(0.5) * (MU(0, 0) + MU(1, 0));
     real sx0 = one, sx1 = one, sy0 = one, sy1 = one;
     if (slope) {
-        sx0 = fmax(one - fabs(PHB(j, i) - PHB(j, i - 1)) / dzthr_x, zero);
-        sx1 = fmax(one - fabs(PHB(j, i + 1) - PHB(j, i)) / dzthr_x, zero);
-        sy0 = fmax(one - fabs(PHB(j, i) - PHB(j - 1, i)) / dzthr_y, zero);
-        sy1 = fmax(one - fabs(PHB(j + 1, i) - PHB(j, i)) / dzthr_y, zero);
+        sx0 = fmax(one - fabs(PHB(0, 0) - PHB(0, -1)) / dzthr_x, zero);
+        sx1 = fmax(one - fabs(PHB(0, 1) - PHB(0, 0)) / dzthr_x, zero);
+        sy0 = fmax(one - fabs(PHB(0, 0) - PHB(-1, 0)) / dzthr_y, zero);
+        sy1 = fmax(one - fabs(PHB(1, 0) - PHB(0, 0)) / dzthr_y, zero);
     }
     const real c1 = d.c1h[k], c2 = d.c2h[k];
     const real cx1 = sx1 * (c1 * mx1 + c2), cx0 = sx0 * (c1 * mx0 + c2);
@@ -1898,8 +1933,8 @@ __global__ void k_diff6q(Dom d, D6Q q, real coef, int mono, int slope,
 #pragma unroll
     for (int e = 0; e < NS; ++e) {
         const real* f = q.f[e];
-        auto FX = [&](int m) { return f[((size_t)k * ny + j) * nx + pmod(i + m, nx)]; };
-        auto FY = [&](int m) { return f[((size_t)k * ny + pmod(j + m, ny)) * nx + i]; };
+        auto FX = [&](int m) { return f[((size_t)k * ny + j) * nx + ix[m + 3]]; };
+        auto FY = [&](int m) { return f[((size_t)k * ny + iy[m + 3]) * nx + i]; };
         real px0 = ten * (FX(0) - FX(-1)) - five * (FX(1) - FX(-2)) + (FX(2) - FX(-3));
         real px1 = ten * (FX(1) - FX(0)) - five * (FX(2) - FX(-1)) + (FX(3) - FX(-2));
         real py0 = ten * (FY(0) - FY(-1)) - five * (FY(1) - FY(-2)) + (FY(2) - FY(-3));
