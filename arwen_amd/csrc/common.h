@@ -188,10 +188,38 @@ __device__ __forceinline__ real flux3(real qm2, real qm1, real q0,
     return div_const(vel * a + fabs(vel) * b, 1.0 / 12.0, R(12.0));
 }
 
-// x**GAMMA evaluated in double and rounded once.
+// x**GAMMA evaluated in double and rounded once.  The general pow is some
+// 200 instructions (us a launch with it and with the form below: k_eos 139
+// and 122 at 523x516x40, k_omega with its EOS stage 286 and 216 at
+// 1000x1000x50).  The FP32 build forms
+//   x^GAMMA = x^2 s^3 x^e,  s = x^(-1/5), e = GAMMA - 7/5 = -2.4e-8,
+// s from the hardware's float log2/exp2 and one step of the series of
+// (1 - h)^(-1/5), h = 1 - x s^5 (|h| < 2e-5, next term 11/125 h^3 < 1e-15),
+// x^e from 1 + z + z^2/2, z = e ln x.  On [2^-16, 16] the error, mostly the
+// float logarithm's in z, stays below 512 double ulps, so a value at least
+// 1024 of them from a float rounding midpoint rounds as the exact one does;
+// the others (one in 2^18) and every other x take pow.
 __device__ __forceinline__ real pow_gamma(real x)
 {
+#if ARW_F64
     return (real)pow((double)x, (double)GAMMA_F);
+#else
+    const float t = __builtin_amdgcn_logf(x);
+    const double s0 = (double)__builtin_amdgcn_exp2f(-0.2f * t);
+    const double X = (double)x;
+    const double s2 = s0 * s0, s5 = (s2 * s2) * s0;
+    const double h = __builtin_fma(-X, s5, 1.0);
+    const double s = __builtin_fma(s0 * h, __builtin_fma(h, 3.0 / 25.0, 0.2), s0);
+    const double z = (double)t * (((double)GAMMA_F - 1.4) * 0.69314718055994531);
+    const double y7 = (X * X) * ((s * s) * s);
+    const double y = __builtin_fma(y7, __builtin_fma(0.5 * z, z, z), y7);
+    const unsigned low = (unsigned)__builtin_bit_cast(unsigned long long, y)
+                         & 0x1fffffffu;
+    const bool fast = x >= 0x1p-16f && x <= 16.0f
+                      && low - (0x10000000u - 1024u) > 2048u;
+    if (fast) return (real)y;
+    return (real)pow(X, (double)GAMMA_F);
+#endif
 }
 
 // The EOS of one cell in perturbation-from-base form (the precision form).
