@@ -27,8 +27,8 @@ struct Batch {
 // Workgroups one member needs in each batched launch shape.  BK_COLT is
 // the column solve's: col_tile columns per workgroup (64, 128 or 256,
 // chosen per ensemble); BK_TILE's workgroups take 64 columns in four level
-// groups; the other column launches keep 256.
-enum BatchKind { BK_COLS, BK_ROWS, BK_TILE, BK_COLT, BK_COUNT };
+// groups, BK_TILE16's the column tile's 16; the other column launches keep 256.
+enum BatchKind { BK_COLS, BK_ROWS, BK_TILE, BK_TILE16, BK_COLT, BK_COUNT };
 int batch_blocks(const Dom& d, int kind, int col_tile);
 
 // The members' views for one launch role, with the per-shape tables.

@@ -1805,17 +1805,24 @@ enum { X_RLO, X_PLO, X_RHI, X_PHI, X_A, X_B, X_C, X_N };
 enum { CF_C1H, CF_C2H, CF_C1F, CF_C2F, CF_DNW, CF_RDNW, CF_RDN, CF_FNM, CF_FNP,
        CF_N };
 
-template <bool B3, bool DAMP, bool AL, bool WW, bool PREC, bool XO, int TX,
-          int L>
-__global__ __launch_bounds__(512) void k_column_tile(Dom d, Sc s, real* RS pout)
+// Batched (Many): the new p'' goes to each member's p_pp_old; the LDS and the
+// level groups are those of the tallest member.
+template <class SRC, bool B3, bool DAMP, bool AL, bool WW, bool PREC, bool XO,
+          int TX, int L>
+__global__ __launch_bounds__(512) void k_column_tile(typename SRC::Arg a_, Sc s,
+                                                     real* RS pout_arg)
 {
+    int m_, g_;
+    if (!SRC::locate(a_, m_, g_)) return;            // the whole workgroup
+    const Dom& d = SRC::dom(a_, m_);
+    real* RS pout = SRC::many ? d.p_pp_old : pout_arg;
     typedef typename std::conditional<PREC, double, real>::type tri;
     constexpr int S = TX;
     struct alignas(4 * sizeof(tri)) Row { tri w, g, a, b; };
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int nz = d.nz, ny = d.ny, nx = d.nx, st = ny * nx;
     const int stu = ny * (nx + 1), stv = (ny + 1) * nx;
-    const int tile = xcd_block() * TX;
+    const int tile = (SRC::many ? g_ : xcd_block()) * TX;
     if (tile >= st) return;                          // the whole workgroup
     const int x = (int)threadIdx.x;
     const int wv = (int)threadIdx.y;
@@ -3200,9 +3207,11 @@ static inline size_t park_bytes(const Sc& c, int cols_per_block)
 // the tile's serial steps and its 4 waves a SIMD cost more.  us a launch,
 // k_column -> k_column_tile: 512 columns x 64 levels 109 -> 14, 3072x30
 // 52 -> 15, 30720x50 (moist) 103 -> 41, 25883x45 (terrain, FP64) 141 -> 75,
-// 50000x49 (terrain) 102 -> 86; but 243987x50 (precision form) 320 -> 428 and
-// 1000000x50 1047 -> 1285.
-constexpr int kTileColumns = 96 * 1024;
+// 50000x49 (terrain) 102 -> 86; us a step 70200x50 1725 -> 1624, an ensemble
+// of four members with 36500 columns together 1415 -> 1027; but 90000x50
+// 1992 -> 2300 (terrain 2454 -> 2887, precision form 2307 -> 2655), 84000x45
+// FP64 3594 -> 4013, 1000000x50 1047 -> 1285 us a launch.
+constexpr int kTileColumns = 72 * 1024;
 constexpr int kTileX = 16, kTileLevels = 4;
 
 // The tile's launch for nz levels: 16 columns keep a workgroup at 4 waves
@@ -3230,17 +3239,16 @@ static bool column_tile(int cols, int nz, bool prec, ColTile& t)
     return cols <= kTileColumns && ng * kTileX <= 512;
 }
 
-template <bool B3, bool DAMP, bool AL, bool WW, bool PREC, bool XO>
-static void launch_column_tile(const Dom& d, const Sc& s0, real* pout,
-                               const ColTile& t, hipStream_t st)
+template <class SRC, bool B3, bool DAMP, bool AL, bool WW, bool PREC, bool XO>
+static void launch_column_tile(const typename SRC::Arg& a, dim3 g, const Sc& s0,
+                               real* pout, const ColTile& t, hipStream_t st)
 {
     Sc s = s0;
     s.lds_rows = t.rows;
     s.lds_groups = t.groups;
-    const dim3 g(xcd_grid((unsigned)(d.ny * d.nx + kTileX - 1) / kTileX));
-    hipLaunchKernelGGL((k_column_tile<B3, DAMP, AL, WW, PREC, XO, kTileX,
+    hipLaunchKernelGGL((k_column_tile<SRC, B3, DAMP, AL, WW, PREC, XO, kTileX,
                                       kTileLevels>),
-                       g, t.block, t.lds, st, d, s, pout);
+                       g, t.block, t.lds, st, a, s, pout);
 }
 
 template <bool B3, bool DAMP, bool AL, bool WW>
@@ -3249,13 +3257,15 @@ static void launch_column(const Dom& d, const Sc& s0, real* pout,
 {
     ColTile t;
     if (column_tile(d.ny * d.nx, d.nz, s0.prec, t)) {
+        const dim3 g = tiles(d, kTileX);
         if (xo_active(d, s0))
             with_prec(s0.prec, [&](auto p) {
-                launch_column_tile<B3, DAMP, AL, WW, decltype(p)::value, true>(
-                    d, s0, pout, t, st);
+                launch_column_tile<One, B3, DAMP, AL, WW, decltype(p)::value,
+                                   true>(d, g, s0, pout, t, st);
             });
         else
-            launch_column_tile<B3, DAMP, AL, WW, false, false>(d, s0, pout, t, st);
+            launch_column_tile<One, B3, DAMP, AL, WW, false, false>(d, g, s0, pout,
+                                                                    t, st);
         return;
     }
     const Sc s = column_sc(s0);
@@ -3369,6 +3379,7 @@ int batch_blocks(const Dom& d, int kind, int col_tile)
     case BK_COLS: return (d.ny * d.nx + 255) / 256;
     case BK_COLT: return (d.ny * d.nx + col_tile - 1) / col_tile;
     case BK_ROWS: return rows;
+    case BK_TILE16: return (d.ny * d.nx + kTileX - 1) / kTileX;
     default: return (d.ny * d.nx + 63) / 64;
     }
 }
@@ -3432,8 +3443,19 @@ hipError_t run_uv_b(const BatchSet& b, const Sc& s, bool b3, hipStream_t st)
 }
 
 template <bool B3, bool DAMP, bool AL>
-static void launch_column_b(const Batch& r, const Sc& s0, hipStream_t st)
+static void launch_column_b(const BatchSet& b, const Sc& s0, hipStream_t st)
 {
+    // the members' columns together fill the chip as one domain's do
+    ColTile t;
+    const Batch& q = b.k[BK_TILE16];
+    if (column_tile(q.total * kTileX, q.nz, s0.prec, t)) {
+        with_prec(s0.prec, [&](auto p) {
+            launch_column_tile<Many, B3, DAMP, AL, false, decltype(p)::value, true>(
+                q, bgrid(q), s0, nullptr, t, st);
+        });
+        return;
+    }
+    const Batch& r = b.k[BK_COLT];
     const Sc s = column_sc(s0);
     const size_t lds = park_bytes(s, r.tile);
     if (s.prec)
@@ -3445,22 +3467,21 @@ static void launch_column_b(const Batch& r, const Sc& s0, hipStream_t st)
 }
 
 template <bool B3, bool DAMP>
-static void launch_column_b_al(const Batch& r, const Sc& s, int al,
+static void launch_column_b_al(const BatchSet& b, const Sc& s, int al,
                                hipStream_t st)
 {
-    if (al) launch_column_b<B3, DAMP, true>(r, s, st);
-    else launch_column_b<B3, DAMP, false>(r, s, st);
+    if (al) launch_column_b<B3, DAMP, true>(b, s, st);
+    else launch_column_b<B3, DAMP, false>(b, s, st);
 }
 
 hipError_t run_column_b(const BatchSet& b, const Sc& s, bool b3, int write_al,
                         hipStream_t st)
 {
-    const Batch& r = b.k[BK_COLT];
     const bool damp = s.damp != 0;
-    if (b3 && damp) launch_column_b_al<true, true>(r, s, write_al, st);
-    else if (b3) launch_column_b_al<true, false>(r, s, write_al, st);
-    else if (damp) launch_column_b_al<false, true>(r, s, write_al, st);
-    else launch_column_b_al<false, false>(r, s, write_al, st);
+    if (b3 && damp) launch_column_b_al<true, true>(b, s, write_al, st);
+    else if (b3) launch_column_b_al<true, false>(b, s, write_al, st);
+    else if (damp) launch_column_b_al<false, true>(b, s, write_al, st);
+    else launch_column_b_al<false, false>(b, s, write_al, st);
     return hipGetLastError();
 }
 
