@@ -303,11 +303,12 @@ struct PgfWin {
 // (dycore.cu:98-157), constant-K diffusion (diffusion.cu:22-51), and the
 // u''/v'' small-step initialisation (dycore.cu:947-1010).  The periodic
 // duplicate faces (u at i = nx, v at j = ny) take the tendency of face 0,
-// whose stencil inputs are theirs, and start from their own u, u0 (v, v0), in
-// the threads of column i = 0 (row j = 0).  PREC (precision form): the
-// pressure gradient takes p' from the perturbation-form EOS.
+// whose stencil inputs are theirs, and start from their own u, u0 (v, v0): with
+// FOLD in the threads of column i = 0 (row j = 0), else in k_tend_faces_edge.
+// PREC (precision form): the pressure gradient takes p' from the
+// perturbation-form EOS.
 template <class SRC, bool B3, bool DIFF, bool PREC, bool HELD = false,
-          bool XO = true>
+          bool XO = true, bool FOLD = true>
 __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
 {
     int m, g;
@@ -596,18 +597,45 @@ __global__ __launch_bounds__(256) void k_tend_faces(typename SRC::Arg a, Sc s)
         win_shift(S, k, rS, cC);
         // the duplicate faces nx, ny: the tendency of face 0, their own
         // u, u0 (last, so that the level above stays one block)
-        if (i == 0) {
+        if (FOLD && i == 0) {
             gst(d.ru_t, lu + j * pu + nx, cC, tu);
             gst(d.u_pp, lu + j * pu + nx, cC,
                 (c1 * mtf_u + c2) * gld(d.u0, lu + j * pu + nx, cC)
                     - (c1 * msf_u + c2) * u_dup);
         }
-        if (j == 0) {
+        if (FOLD && j == 0) {
             gst(d.rv_t, lv + ny * nx, cC, tv);
             gst(d.v_pp, lv + ny * nx, cC,
                 (c1 * mtf_v + c2) * gld(d.v0, lv + ny * nx, cC)
                     - (c1 * msf_v + c2) * v_dup);
         }
+    }
+}
+
+// The duplicate faces of a large domain, after k_tend_faces without FOLD: one
+// thread per (k, j) face u(nx) and per (k, i) face v(ny).
+__global__ __launch_bounds__(256) void k_tend_faces_edge(Dom d)
+{
+    const int nz = d.nz, ny = d.ny, nx = d.nx, pu = nx + 1;
+    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    // mass columns A (of face 0) and B (across it), faces f0 and fd
+    auto face = [&](real* rt, real* pp, const real* x0, const real* x, int k,
+                    int cA, int cB, int f0, int fd) {
+        const real msA = d.mub2d[cA] + d.mup[cA], msB = d.mub2d[cB] + d.mup[cB];
+        const real mtA = d.mub2d[cA] + d.mup0[cA], mtB = d.mub2d[cB] + d.mup0[cB];
+        const real mt = R(0.5) * (mtA + mtB), ms = R(0.5) * (msA + msB);
+        const real c1 = d.c1h[k], c2 = d.c2h[k];
+        rt[fd] = rt[f0];
+        pp[fd] = (c1 * mt + c2) * x0[fd] - (c1 * ms + c2) * x[fd];
+    };
+    if (t < nz * ny) {
+        const int k = t / ny, j = t - k * ny;
+        const int f0 = (k * ny + j) * pu;
+        face(d.ru_t, d.u_pp, d.u0, d.u, k, j * nx, j * nx + nx - 1, f0, f0 + nx);
+    } else if (t < nz * (ny + nx)) {
+        const int r = t - nz * ny, k = r / nx, i = r - k * nx;
+        const int f0 = k * (ny + 1) * nx + i;
+        face(d.rv_t, d.v_pp, d.v0, d.v, k, i, (ny - 1) * nx + i, f0, f0 + ny * nx);
     }
 }
 
@@ -3014,20 +3042,20 @@ static void with_prec(bool prec, F&& f)
 // words per point at 1000x1000x50) and the kernel runs slower.
 constexpr size_t kTendFacesLds = 40 * 1024;
 
-template <class SRC, bool PREC, bool XO = true>
+template <class SRC, bool PREC, bool XO = true, bool FOLD = true>
 static void launch_tend_faces(const typename SRC::Arg& a, dim3 g, const Sc& s,
                               bool b3, hipStream_t st)
 {
     const dim3 b(64, 4);
     const size_t l = kTendFacesLds;
     if (b3 && s.diff)
-        hipLaunchKernelGGL((k_tend_faces<SRC, true, true, PREC, false, XO>), g, b, l, st, a, s);
+        hipLaunchKernelGGL((k_tend_faces<SRC, true, true, PREC, false, XO, FOLD>), g, b, l, st, a, s);
     else if (b3)
-        hipLaunchKernelGGL((k_tend_faces<SRC, true, false, PREC, false, XO>), g, b, l, st, a, s);
+        hipLaunchKernelGGL((k_tend_faces<SRC, true, false, PREC, false, XO, FOLD>), g, b, l, st, a, s);
     else if (s.diff)
-        hipLaunchKernelGGL((k_tend_faces<SRC, false, true, PREC, false, XO>), g, b, l, st, a, s);
+        hipLaunchKernelGGL((k_tend_faces<SRC, false, true, PREC, false, XO, FOLD>), g, b, l, st, a, s);
     else
-        hipLaunchKernelGGL((k_tend_faces<SRC, false, false, PREC, false, XO>), g, b, l, st, a, s);
+        hipLaunchKernelGGL((k_tend_faces<SRC, false, false, PREC, false, XO, FOLD>), g, b, l, st, a, s);
 }
 
 template <class SRC, bool MOIST, bool PREC, bool XO = true>
@@ -3103,6 +3131,32 @@ static unsigned stencil_groups(unsigned blocks, int nz)
     return few > most ? few : most;
 }
 
+// k_tend_faces without options, from this many workgroups on, leaves the
+// duplicate faces to a launch of their own: the conditional stores at the end of
+// every level cost each wave more than the launch does.  us of both launches
+// against folded: 1000x1000x50 938 and 978, 640x640x64 507 and 520, 700x700x30
+// 310 and 317, terrain 700x700x50 538 and 550, 460x460x50 246 and 252; 400x400x50
+// (700 workgroups) 188 and 190, 250x200x49 terrain 61 and 59, 64x48x30 16 and 12.
+// With the options live the body hides them: 1000x1000x50 with six species 1001
+// and 990; so it does in FP64: 500x500x50 10.94 and 10.47 ms a step.  A launch
+// that just fills the CUs' four slots (kTendFacesLds) is not split either:
+// 500x500x50 257 against 268 in six groups, 512x512x50 253 and 271.
+constexpr unsigned kTendFacesApart = 768;
+
+static bool tend_faces_apart(const Dom& d, const Sc& s, dim3 g, hipStream_t st)
+{
+#if ARW_F64
+    return false;
+#else
+    if (g.x < kTendFacesApart) return false;
+    if (g.x > 15 * 64 && g.x <= 4 * 256) g.y = 1;
+    launch_tend_faces<One, false, false, false>(d, g, s, d.base3d != 0, st);
+    const int n = d.nz * (d.ny + d.nx);
+    hipLaunchKernelGGL(k_tend_faces_edge, dim3((n + 255) / 256), dim3(256), 0, st, d);
+    return true;
+#endif
+}
+
 hipError_t run_tend_faces(const Dom& d, const Sc& s, hipStream_t st)
 {
     dim3 g = rowseg_grid(d.nx, d.ny);
@@ -3117,7 +3171,7 @@ hipError_t run_tend_faces(const Dom& d, const Sc& s, hipStream_t st)
         with_prec(s.prec, [&](auto p) {
             launch_tend_faces<One, decltype(p)::value>(d, g, s, b3, st);
         });
-    } else {
+    } else if (!tend_faces_apart(d, s, g, st)) {
         launch_tend_faces<One, false, false>(d, g, s, b3, st);
     }
     return hipGetLastError();

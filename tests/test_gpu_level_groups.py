@@ -64,6 +64,22 @@ def test_step_is_bit_identical_at_the_edges_of_the_launch_shapes(kind, size):
         assert same == 1.0, f"{n}: rel {err:.3e}, {same:.6f} identical"
 
 
+# 768 workgroups of 64 x 4 columns and 975, 1046: the duplicate faces in a
+# launch of their own, the levels in one group and in several
+@pytest.mark.parametrize("kind", ["flat", "terrain", "diffusion"])
+@pytest.mark.parametrize("size", [(3, 3070, 5), (2, 3900, 5), (65, 2091, 4)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_duplicate_faces_launched_apart(kind, size):
+    from arwen_amd import dycore
+    case = _case(kind, *size)
+    o, g = oracle_and_gpu(case)
+    O.step(o, case.cfg)
+    dycore.step(g, case.cfg)
+    for n, (err, same) in compare(o, g, PROG + DIAG).items():
+        assert np.all(np.isfinite(getattr(o, n))), n
+        assert same == 1.0, f"{n}: rel {err:.3e}, {same:.6f} identical"
+
+
 @pytest.mark.parametrize("size", [(5, 3, 3), (17, 9, 128), (131, 127, 9)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_precision_form_is_bit_identical_there(size):
