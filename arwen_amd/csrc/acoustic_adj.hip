@@ -245,7 +245,8 @@ constexpr int S1_TX = 16;
 __global__ __launch_bounds__(256) void k_adj_s1_lu(Dom d, Fw f, const real* lu)
 {
     struct alignas(4 * sizeof(real)) Row { real v, gp, al, a; };
-    extern __shared__ __align__(16) unsigned char s1_lds[];
+    static_assert(alignof(Row) <= kLdsAlign, "rows over s1_lds");
+    extern __shared__ ARW_LDS_ALIGN unsigned char s1_lds[];
     Row* const L = reinterpret_cast<Row*>(s1_lds) + threadIdx.x;
     const int st = d.ny * d.nx, nz = d.nz;
     const int c0 = (int)xcd_block() * S1_TX + (int)threadIdx.x;

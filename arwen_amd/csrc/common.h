@@ -376,6 +376,11 @@ struct Kahan {
     }
 };
 
+// Alignment of a dynamic LDS buffer that rows of four values are laid over
+// (read and written with one instruction): four doubles.
+#define ARW_LDS_ALIGN __align__(32)
+constexpr size_t kLdsAlign = 32;
+
 // Column sums split over KG level groups: thread (tx, ty) of a (64, KG)
 // block sums levels ty, ty + KG, ... of column blockIdx.x * 64 + tx (each
 // level's loads coalesced over tx), then the groups meet in LDS.  Four

@@ -123,7 +123,7 @@ __device__ __forceinline__ TileCol tile_col(int tile, int st, int nz)
 template <class SRC, bool EOS, bool B3, bool PREC, bool XO, int TX>
 __global__ __launch_bounds__(256) void k_omega(typename SRC::Arg a, Sc s)
 {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
+    extern __shared__ ARW_LDS_ALIGN unsigned char lds_raw[];
     int m, g;
     if (!SRC::locate(a, m, g)) return;
     const Dom& d = SRC::dom(a, m);
@@ -1847,7 +1847,8 @@ __global__ __launch_bounds__(512) void k_column_tile(typename SRC::Arg a_, Sc s,
     typedef typename std::conditional<PREC, double, real>::type tri;
     constexpr int S = TX;
     struct alignas(4 * sizeof(tri)) Row { tri w, g, a, b; };
-    extern __shared__ __align__(16) unsigned char lds_raw[];
+    static_assert(alignof(Row) <= kLdsAlign, "rows over lds_raw");
+    extern __shared__ ARW_LDS_ALIGN unsigned char lds_raw[];
     const int nz = d.nz, ny = d.ny, nx = d.nx, st = ny * nx;
     const int stu = ny * (nx + 1), stv = (ny + 1) * nx;
     const int tile = (SRC::many ? g_ : xcd_block()) * TX;
