@@ -144,3 +144,40 @@ def test_precision_form_ensemble_matches_member_steps_bitwise(terrain):
         ens.step(2)
     torch.cuda.synchronize()
     _assert_same(seq, ens_states)
+
+
+@pytest.mark.parametrize("tile", [64, 128, 256])
+@pytest.mark.parametrize("form", ["flat", "terrain", "precision",
+                                  "precision terrain", "fp64", "fp64 terrain"])
+def test_column_march_ensemble_matches_member_steps_bitwise(form, tile):
+    """A member of 130 levels (flat: and one of 260, more than the batched
+    Omega's LDS holds) is more than a column tile takes, so the ensemble's
+    column solve is k_column with col_tile columns a workgroup; the members
+    stepped alone take the column tile but for the tall ones."""
+    from arwen_amd import dycore
+    from arwen_amd.ensemble import Ensemble
+    from arwen_amd.state import DomainState
+    shapes = SHAPES[:3] + [(21, 13, 130)] + [(9, 7, 260)] * (form == "flat")
+    dtype = torch.float64 if "fp64" in form else torch.float32
+    print(f"ensemble column march {form} col_tile={tile}", flush=True)
+
+    def states():
+        out = []
+        for i, (nx, ny, nz) in enumerate(shapes):
+            case = (cases.stratified_hill(nx=nx, ny=ny, nz=nz, seed=100 + i,
+                                          radius=20000.0)
+                    if "terrain" in form
+                    else cases.ensemble_member(nx, ny, nz, seed=100 + i))
+            st = DomainState.from_host(case, dtype=dtype)
+            st.cfg = st.cfg.with_(precision_form="precision" in form)
+            out.append(st)
+        return out
+
+    seq, ens_states = states(), states()
+    for st in seq:
+        dycore.run_steps(st, st.cfg, 2)
+    with Ensemble(ens_states, seq[0].cfg, col_tile=tile) as ens:
+        ens.step(2)
+    torch.cuda.synchronize()
+    _assert_same(seq, ens_states)
+    assert all(bool(torch.isfinite(st.p).all()) for st in seq)

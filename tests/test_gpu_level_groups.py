@@ -107,3 +107,61 @@ def test_fp64_build_agrees_there(size):
     # pow's last bit, 2e-16 of a pressure whose differences the step takes
     for n, (err, _) in compare(o, g, PROG + DIAG).items():
         assert err < 1e-9, f"{n}: rel {err:.3e}"
+
+
+# more levels than a column tile takes: k_column, whose forms these few columns
+# would otherwise not reach
+@pytest.mark.parametrize("kind", ["terrain", "moist_cq"])
+def test_column_march_options_are_bit_identical(kind):
+    """The precision form over terrain, and moist_cq."""
+    from arwen_amd import dycore
+    if kind == "terrain":
+        case = _case(kind, 3, 70, 130)
+        case.cfg = case.cfg.with_(precision_form=True)
+    else:
+        case = _case("moist", 3, 70, 130)
+        case.cfg = case.cfg.with_(moist_cq=True)
+    o, g = oracle_and_gpu(case)
+    names = PROG + DIAG
+    if kind == "moist_cq":
+        import torch
+        q = ("qv", "qc", "qr") + o.extra
+        names = names + q
+        for n in q + ("h_diabatic",):
+            getattr(g, n).copy_(torch.as_tensor(getattr(o, n)))
+    O.step(o, case.cfg)
+    dycore.step(g, case.cfg)
+    for n, (err, same) in compare(o, g, names).items():
+        assert np.all(np.isfinite(getattr(o, n))), n
+        assert same == 1.0, f"{n}: rel {err:.3e}, {same:.6f} identical"
+
+
+def test_column_march_precision_form_is_bit_identical():
+    test_precision_form_is_bit_identical_there((3, 70, 130))
+
+
+@pytest.mark.parametrize("kind", ["fp64", "terrain"])
+def test_column_march_fp64_agrees(kind):
+    import torch
+    from arwen_amd import dycore
+    from arwen_amd.state import DomainState
+    case = _case(kind, 3, 70, 130)
+    o = O.from_case(case, np.float64)
+    g = DomainState.from_host(case, dtype=torch.float64)
+    O.step(o, case.cfg)
+    dycore.step(g, case.cfg)
+    # as above: pow's last bit
+    for n, (err, _) in compare(o, g, PROG + DIAG).items():
+        assert err < 1e-9, f"{n}: rel {err:.3e}"
+
+
+def test_omega_in_wide_tiles_parks_more_levels_than_its_lds_holds():
+    """Above 16384 columns Omega's tile is 64 columns wide; its LDS holds 256
+    levels of them."""
+    from arwen_amd import dycore
+    case = _case("flat", 129, 128, 257)
+    o, g = oracle_and_gpu(case)
+    O.step(o, case.cfg)
+    dycore.step(g, case.cfg)
+    for n, (err, same) in compare(o, g, PROG + DIAG).items():
+        assert same == 1.0, f"{n}: rel {err:.3e}, {same:.6f} identical"
