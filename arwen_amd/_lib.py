@@ -262,6 +262,7 @@ def load():
         "arw_ensemble_step": ([_P, _I, _P], _I),
         "arw_ensemble_capture": ([_P, _I, _I], _I),
         "arw_ensemble_launch": ([_P, _P], _I),
+        "arw_ensemble_column_tile": ([_P, _P], _I),
         "arw_ensemble_destroy": ([_P], _I),
     }
     flux = [_P, _P, _P, _P, _P, _P, _P, _P, _F, _F, _I, _I, _I, _P]
@@ -317,6 +318,7 @@ FP64_ENTRY_POINTS = (
     "arw64_acoustic_adjoint_work", "arw64_ensemble_create",
     "arw64_ensemble_step",
     "arw64_ensemble_capture", "arw64_ensemble_launch",
+    "arw64_ensemble_column_tile",
     "arw64_ensemble_destroy", "arw64_stage_tendencies_adjoint",
     "arw64_stage_adjoint_work", "arw64_small_step_init_adjoint",
     "arw64_small_step_finish_adjoint", "arw64_small_step_adjoint_work",
@@ -348,7 +350,8 @@ def exported_symbols() -> list[str]:
             "arw_acoustic_substep_adjoint", "arw_acoustic_adjoint_work",
             "arw_ensemble_create",
             "arw_ensemble_step", "arw_ensemble_capture",
-            "arw_ensemble_launch", "arw_ensemble_destroy",
+            "arw_ensemble_launch", "arw_ensemble_column_tile",
+            "arw_ensemble_destroy",
             "arw_stage_tendencies_adjoint", "arw_stage_adjoint_work",
             "arw_small_step_init_adjoint", "arw_small_step_finish_adjoint",
             "arw_small_step_adjoint_work",

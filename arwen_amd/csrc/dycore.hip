@@ -1587,6 +1587,7 @@ enum { ENS_BASE = 9, ENS_ROLES = 10 };
 
 struct EnsGroup {
     BatchSet sets[ENS_ROLES];
+    int cols;              // its members' columns
 };
 
 // The views arw_step's stage loop forms for one member (same rotation).
@@ -1617,8 +1618,9 @@ void member_views(const Dom& d, Dom* role, FinishDst* fin)
 }
 
 // One step of one group: the launch sequence of arw_step, each launch
-// covering every member of the group.
-int32_t ens_issue(const EnsGroup& G, const arw_params* prm, bool b3,
+// covering every member of the group.  cols: columns that run at once, the
+// group's own or those of all groups side by side.
+int32_t ens_issue(const EnsGroup& G, const arw_params* prm, bool b3, int cols,
                   hipStream_t st)
 {
     const int ns = prm->time_step_sound;
@@ -1642,7 +1644,7 @@ int32_t ens_issue(const EnsGroup& G, const arw_params* prm, bool b3,
             const BatchSet& DS = G.sets[3 * stage + 1 + (n & 1)];
             if ((rc = launched(run_uv_b(DS, sn, b3, st), "k_uv (ensemble)", -1, st)))
                 return rc;
-            if ((rc = launched(run_column_b(DS, sn, b3, b3 || last, st), "k_column (ensemble)", -1, st)))
+            if ((rc = launched(run_column_b(DS, sn, b3, b3 || last, cols, st), "k_column (ensemble)", -1, st)))
                 return rc;
         }
         if ((rc = launched(run_finish_b(DD, b3, s.prec != 0, st), "k_finish (ensemble)", -1, st)))
@@ -2004,6 +2006,7 @@ struct ARW_API(ensemble) {
     int n = 0;
     arw_params prm{};
     bool b3 = false;
+    int cols = 0;                         // all members' columns
     void* dev = nullptr;                  // views and work tables
     std::vector<EnsGroup> groups;
     hipGraphExec_t exec = nullptr;
@@ -2985,6 +2988,10 @@ int32_t ARW_API(ensemble_create)(const Dom* members, int32_t n,
     e->groups.resize(groups);
     for (int g = 0; g < groups; ++g) {
         const size_t ng = gm[g].size();
+        long long gc = 0;
+        for (int m : gm[g]) gc += (long long)members[m].ny * members[m].nx;
+        e->groups[g].cols = (int)std::min(gc, 1LL << 30);
+        e->cols = (int)std::min(gc + e->cols, 1LL << 30);
         for (int r = 0; r < ENS_ROLES; ++r) {
             const int stage = r < ENS_BASE ? r / 3 : -1;
             for (int k = 0; k < BK_COUNT; ++k) {
@@ -3014,7 +3021,7 @@ int32_t ARW_API(ensemble_step)(ARW_API(ensemble)* e, int32_t nsteps,
     hipStream_t st = (hipStream_t)stream;
     for (int t = 0; t < nsteps; ++t)
         for (const EnsGroup& G : e->groups) {
-            int32_t rc = ens_issue(G, &e->prm, e->b3, st);
+            int32_t rc = ens_issue(G, &e->prm, e->b3, G.cols, st);
             if (rc) return rc;
         }
     return ARW_OK;
@@ -3060,7 +3067,7 @@ int32_t ARW_API(ensemble_capture)(ARW_API(ensemble)* e, int32_t nsteps,
         }
         for (int g = 0; g < ng && rc == ARW_OK; ++g)
             for (int t = 0; t < nt && rc == ARW_OK; ++t)
-                rc = ens_issue(e->groups[g], &e->prm, e->b3, cs[g]);
+                rc = ens_issue(e->groups[g], &e->prm, e->b3, e->cols, cs[g]);
         // join
         for (int g = 1; g < ng && rc == ARW_OK; ++g)
             if (hipEventRecord(ev[g], cs[g]) != hipSuccess
@@ -3081,6 +3088,16 @@ int32_t ARW_API(ensemble_capture)(ARW_API(ensemble)* e, int32_t nsteps,
         if (cs[g]) hipStreamDestroy(cs[g]);
     }
     return rc;
+}
+
+int32_t ARW_API(ensemble_column_tile)(const ARW_API(ensemble)* e, int32_t* columns)
+{
+    if (!e || !columns) return fail(ARW_E_ARG, "null argument");
+    bool tiled = true;
+    for (const EnsGroup& G : e->groups)
+        tiled = tiled && column_tiled(G.sets[1], e->prm.precision_form != 0, e->cols);
+    *columns = tiled ? 16 : e->groups[0].sets[1].k[BK_COLT].tile;
+    return ARW_OK;
 }
 
 int32_t ARW_API(ensemble_launch)(ARW_API(ensemble)* e, void* stream)

@@ -3498,12 +3498,15 @@ hipError_t run_uv_b(const BatchSet& b, const Sc& s, bool b3, hipStream_t st)
 }
 
 template <bool B3, bool DAMP, bool AL>
-static void launch_column_b(const BatchSet& b, const Sc& s0, hipStream_t st)
+static void launch_column_b(const BatchSet& b, const Sc& s0, int cols,
+                            hipStream_t st)
 {
-    // the members' columns together fill the chip as one domain's do
+    // the columns of all members that run at once fill the chip as one
+    // domain's do: ten members of 239 907 columns in four groups take 11.95 ms
+    // for two steps when each group's 60 000 are tiled, 11.25 when none is
     ColTile t;
     const Batch& q = b.k[BK_TILE16];
-    if (column_tile(q.total * kTileX, q.nz, s0.prec, t)) {
+    if (column_tile(cols, q.nz, s0.prec, t)) {
         with_prec(s0.prec, [&](auto p) {
             launch_column_tile<Many, B3, DAMP, AL, false, decltype(p)::value, true>(
                 q, bgrid(q), s0, nullptr, t, st);
@@ -3522,21 +3525,27 @@ static void launch_column_b(const BatchSet& b, const Sc& s0, hipStream_t st)
 }
 
 template <bool B3, bool DAMP>
-static void launch_column_b_al(const BatchSet& b, const Sc& s, int al,
+static void launch_column_b_al(const BatchSet& b, const Sc& s, int al, int cols,
                                hipStream_t st)
 {
-    if (al) launch_column_b<B3, DAMP, true>(b, s, st);
-    else launch_column_b<B3, DAMP, false>(b, s, st);
+    if (al) launch_column_b<B3, DAMP, true>(b, s, cols, st);
+    else launch_column_b<B3, DAMP, false>(b, s, cols, st);
+}
+
+bool column_tiled(const BatchSet& b, bool prec, int cols)
+{
+    ColTile t;
+    return column_tile(cols, b.k[BK_TILE16].nz, prec, t);
 }
 
 hipError_t run_column_b(const BatchSet& b, const Sc& s, bool b3, int write_al,
-                        hipStream_t st)
+                        int cols, hipStream_t st)
 {
     const bool damp = s.damp != 0;
-    if (b3 && damp) launch_column_b_al<true, true>(b, s, write_al, st);
-    else if (b3) launch_column_b_al<true, false>(b, s, write_al, st);
-    else if (damp) launch_column_b_al<false, true>(b, s, write_al, st);
-    else launch_column_b_al<false, false>(b, s, write_al, st);
+    if (b3 && damp) launch_column_b_al<true, true>(b, s, write_al, cols, st);
+    else if (b3) launch_column_b_al<true, false>(b, s, write_al, cols, st);
+    else if (damp) launch_column_b_al<false, true>(b, s, write_al, cols, st);
+    else launch_column_b_al<false, false>(b, s, write_al, cols, st);
     return hipGetLastError();
 }
 

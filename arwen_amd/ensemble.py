@@ -122,6 +122,15 @@ class Ensemble:
         for st in self.states:
             st.elapsed_seconds += self.graph_steps * self.cfg.dt
 
+    @property
+    def column_tile(self) -> int:
+        """Columns per workgroup of a captured graph's column solve: 16
+        where the members' columns are few, else ``col_tile``."""
+        name, fn = self._fn("ensemble_column_tile")
+        out = ctypes.c_int32()
+        _lib.check(fn(self._h, ctypes.byref(out)), name)
+        return out.value
+
     def close(self) -> None:
         if self._h is not None:
             torch.cuda.synchronize()

@@ -326,7 +326,8 @@ int32_t arw_tracer_adjoint(const arw_domain *d, const arw_params *prm,
  *         work; each group is its own launch sequence, and a captured
  *         graph runs the groups as parallel branches (1 <= groups <= n).
  * col_tile: columns per workgroup of the batched column solve (64, 128
- *         or 256; results do not depend on it).
+ *         or 256; results do not depend on it).  It has no effect where
+ *         the members' columns are few: the solve then takes tiles of 16.
  * The handle owns its device tables until arw_ensemble_destroy.
  */
 typedef struct arw_ensemble arw_ensemble;
@@ -343,6 +344,9 @@ int32_t arw_ensemble_step(arw_ensemble *e, int32_t nsteps, void *stream);
 int32_t arw_ensemble_capture(arw_ensemble *e, int32_t nsteps,
                              int32_t join_every);
 int32_t arw_ensemble_launch(arw_ensemble *e, void *stream);
+/* *columns: columns per workgroup of the captured graph's column solve, 16
+ * or create's col_tile (where groups differ, col_tile). */
+int32_t arw_ensemble_column_tile(const arw_ensemble *e, int32_t *columns);
 int32_t arw_ensemble_destroy(arw_ensemble *e);
 
 /*
@@ -916,6 +920,8 @@ int32_t arw64_ensemble_step(arw64_ensemble *e, int32_t nsteps,
 int32_t arw64_ensemble_capture(arw64_ensemble *e, int32_t nsteps,
                                int32_t join_every);
 int32_t arw64_ensemble_launch(arw64_ensemble *e, void *stream);
+int32_t arw64_ensemble_column_tile(const arw64_ensemble *e,
+                                   int32_t *columns);
 int32_t arw64_ensemble_destroy(arw64_ensemble *e);
 
 #ifdef __cplusplus

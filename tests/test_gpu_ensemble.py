@@ -181,3 +181,47 @@ def test_column_march_ensemble_matches_member_steps_bitwise(form, tile):
     torch.cuda.synchronize()
     _assert_same(seq, ens_states)
     assert all(bool(torch.isfinite(st.p).all()) for st in seq)
+
+
+@pytest.mark.parametrize("members,groups,tile", [(2, 1, 16), (2, 2, 16),
+                                                 (4, 1, 128), (4, 2, 128)])
+def test_column_tile_counts_all_groups_columns(members, groups, tile):
+    """A captured graph's groups run side by side, so the column solve is
+    chosen by the columns of all of them: 39 000 take 16-column tiles, 78 000
+    in two groups take k_column like 78 000 in one."""
+    from arwen_amd import dycore
+    from arwen_amd.ensemble import Ensemble
+    from arwen_amd.state import DomainState
+    states = [[DomainState.from_host(cases.ensemble_member(150, 130, 8,
+                                                           seed=7 + i))
+               for i in range(members)] for _ in range(2)]
+    print(f"ensemble column tile members={members} groups={groups}",
+          flush=True)
+    for st in states[0]:
+        dycore.run_steps(st, st.cfg, 1)
+    with Ensemble(states[1], states[1][0].cfg, groups=groups,
+                  col_tile=128) as ens:
+        assert ens.column_tile == tile
+        ens.capture(1)
+        ens.launch()
+    torch.cuda.synchronize()
+    _assert_same(*states)
+
+
+def test_short_members_in_a_tall_batch():
+    """Members of the fewest levels beside one of 64: level groups without
+    levels in their workgroups."""
+    from arwen_amd import dycore
+    from arwen_amd.ensemble import Ensemble
+    from arwen_amd.state import DomainState
+    states = [[DomainState.from_host(cases.ensemble_member(*sh, seed=3))
+               for sh in ((5, 3, 3), (64, 4, 4), (20, 9, 5), (33, 7, 64))]
+              for _ in range(2)]
+    print("ensemble short members", flush=True)
+    for st in states[0]:
+        dycore.run_steps(st, st.cfg, 2)
+    with Ensemble(states[1], states[1][0].cfg) as ens:
+        assert ens.column_tile == 16
+        ens.step(2)
+    torch.cuda.synchronize()
+    _assert_same(*states)
