@@ -188,9 +188,11 @@ _TUNED: dict = {}
 
 def _time_layout(states, cfg, saved, order, groups, join_every, steps, reps,
                  col_tile=256):
+    """(ms per step, columns per workgroup of the column solve)."""
     with Ensemble(states, cfg, order=order, groups=groups,
                   join_every=join_every, col_tile=col_tile) as ens:
         ens.capture(steps)
+        tile = ens.column_tile
         ens.launch()                               # warm-up replay
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -199,7 +201,7 @@ def _time_layout(states, cfg, saved, order, groups, join_every, steps, reps,
         torch.cuda.synchronize()
         ms = (time.perf_counter() - t0) * 1e3 / (reps * steps)
     restore_state(states, saved)
-    return ms
+    return ms, tile
 
 
 def autotune(states: list[DomainState], cfg: RunConfig, *, steps: int = 10,
@@ -210,7 +212,9 @@ def autotune(states: list[DomainState], cfg: RunConfig, *, steps: int = 10,
     the member order of the work tables (one group), then the number of
     groups that run as parallel graph branches and how often the branches
     rejoin (the substep schedule across the branches), then the column
-    solve's tile (columns per workgroup) for that layout.  Returns
+    solve's tile (columns per workgroup) for that layout; where the members'
+    columns are so few that the solve takes 16 whatever ``col_tile`` says,
+    those trials are the layout's own measurement.  Returns
     {"order", "order_name", "groups", "join_every", "col_tile",
     "ms_per_step", "trials"}; the members' state is restored afterwards
     and the result is cached per member shapes and step parameters."""
@@ -223,11 +227,12 @@ def autotune(states: list[DomainState], cfg: RunConfig, *, steps: int = 10,
     cands = member_orders(states)
     if orders is not None:
         cands = {k: v for k, v in cands.items() if k in orders}
-    trials = []
+    trials, tile_used = [], {}
 
-    def run(oname, g, j, t=256):
-        ms = _time_layout(states, cfg, saved, cands[oname], g, j, steps,
-                          reps, t)
+    def run(oname, g, j, t=256, ms=None):
+        if ms is None:
+            ms, tile_used[oname, g, j] = _time_layout(
+                states, cfg, saved, cands[oname], g, j, steps, reps, t)
         trials.append({"order": oname, "groups": g, "join_every": j,
                        "col_tile": t, "ms_per_step": ms})
         if verbose:
@@ -243,9 +248,11 @@ def autotune(states: list[DomainState], cfg: RunConfig, *, steps: int = 10,
         for j in joins:
             run(best_order, g, j)
     lay = min(trials, key=lambda t: t["ms_per_step"])
+    layout = lay["order"], lay["groups"], lay["join_every"]
+    same = lay["ms_per_step"] if tile_used[layout] != 256 else None
     for t in col_tiles:
         if t != 256:
-            run(lay["order"], lay["groups"], lay["join_every"], t)
+            run(*layout, t, ms=same)
     best = min(trials, key=lambda t: t["ms_per_step"])
     # a trial graph of `steps` steps with join_every = 0 rejoins at its end,
     # i.e. every `steps` steps: that is what was measured, and what a longer

@@ -225,3 +225,23 @@ def test_short_members_in_a_tall_batch():
         ens.step(2)
     torch.cuda.synchronize()
     _assert_same(*states)
+
+
+@pytest.mark.parametrize("tall", [False, True])
+def test_autotune_times_column_tiles_only_where_they_differ(tall, monkeypatch):
+    """Few columns take 16-column tiles whatever col_tile says: the tuner
+    neither times those layouts again nor picks one of them by noise."""
+    from arwen_amd import ensemble as E
+    from arwen_amd.state import DomainState
+    shapes = SHAPES[:2] + [(11, 10, 130 if tall else 13)]
+    states = [DomainState.from_host(cases.ensemble_member(*sh, seed=100))
+              for sh in shapes]
+    timed, time_layout = [], E._time_layout
+    monkeypatch.setattr(E, "_time_layout", lambda *a: (
+        timed.append(a[-1]), time_layout(*a))[1])
+    print(f"ensemble autotune tall={tall}", flush=True)
+    res = E.autotune(states, states[0].cfg, steps=1, reps=1, groups=(1,))
+    assert [t for t in timed if t != 256] == ([128, 64] if tall else [])
+    assert [t["col_tile"] for t in res["trials"]][-2:] == [128, 64]
+    if not tall:
+        assert res["col_tile"] == 256
