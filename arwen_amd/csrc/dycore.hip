@@ -3095,7 +3095,8 @@ int32_t ARW_API(ensemble_column_tile)(const ARW_API(ensemble)* e, int32_t* colum
     if (!e || !columns) return fail(ARW_E_ARG, "null argument");
     bool tiled = true;
     for (const EnsGroup& G : e->groups)
-        tiled = tiled && column_tiled(G.sets[1], e->prm.precision_form != 0, e->cols);
+        tiled = tiled && column_tiled(G.sets[1], e->b3, e->prm.precision_form != 0,
+                                      e->cols);
     *columns = tiled ? 16 : e->groups[0].sets[1].k[BK_COLT].tile;
     return ARW_OK;
 }

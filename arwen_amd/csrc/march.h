@@ -198,7 +198,7 @@ hipError_t run_uv_b(const BatchSet& b, const Sc& s, bool b3, hipStream_t st);
 // cols: the columns of everything that runs at once with this launch (the
 // groups of a captured graph are parallel branches).  column_tiled: whether the
 // column solve then takes the 16-column tile, where BK_COLT has no effect.
-bool column_tiled(const BatchSet& b, bool prec, int cols);
+bool column_tiled(const BatchSet& b, bool b3, bool prec, int cols);
 hipError_t run_column_b(const BatchSet& b, const Sc& s, bool b3, int write_al,
                         int cols, hipStream_t st);
 hipError_t run_finish_b(const BatchSet& b, bool b3, bool prec, hipStream_t st);

@@ -3256,18 +3256,56 @@ static inline size_t park_bytes(const Sc& c, int cols_per_block)
     return (size_t)2 * c.park * cols_per_block * sizeof(real);
 }
 
-// The column solve is tiled up to this many columns.  One thread per column
-// (k_column) then leaves most SIMDs with at most one wave, whose two sweeps
-// wait on one level's loads at a time; beyond it k_column has the waves, and
-// the tile's serial steps and its 4 waves a SIMD cost more.  us a launch,
-// k_column -> k_column_tile: 512 columns x 64 levels 109 -> 14, 3072x30
-// 52 -> 15, 30720x50 (moist) 103 -> 41, 25883x45 (terrain, FP64) 141 -> 75,
-// 50000x49 (terrain) 102 -> 86; us a step 70200x50 1725 -> 1624, an ensemble
-// of four members with 36500 columns together 1415 -> 1027; but 90000x50
-// 1992 -> 2300 (terrain 2454 -> 2887, precision form 2307 -> 2655), 84000x45
-// FP64 3594 -> 4013, 1000000x50 1047 -> 1285 us a launch.
-constexpr int kTileColumns = 72 * 1024;
 constexpr int kTileX = 16, kTileLevels = 4;
+
+// The column solve is tiled up to this many columns of nz levels (b3: terrain;
+// sums: with the scalars' flux sums; many: an ensemble's, nz the tallest's).  One thread per column (k_column) then
+// leaves most SIMDs with at most one wave, whose two sweeps wait on one level's
+// loads at a time; beyond it k_column has the waves, and the tile's serial steps
+// and its 4 waves a SIMD cost more.  More levels and wider rows take more LDS a
+// workgroup, so fewer of them run at once; below 6 levels the tile has more
+// barriers than work.  A step with the tile over one with k_column on the same
+// memory, mean of four allocations:
+//   columns           34K  44K  53K  61K  67K  74K  88K
+//   flat 30 levels    .77  .82  .85  .87  .88  .91 1.02
+//   flat 50           .72  .78  .93  .98 1.29  .95 1.13
+//   flat 64           .70  .85 1.16  .90 1.01 1.03 1.18
+//   terrain 30        .77  .83  .91  .92  .88  .95 1.10
+//   terrain 50        .73  .84 1.06 1.12  .98 1.00 1.14
+//   precision 50      .78  .86 1.00 1.08  .96 1.00 1.05
+//   moist 50          .76  .83  .96 1.02  .95  .95 1.00
+//   moist 64          .75  .88  .90  .89  .90 1.01 1.02
+//   FP64 50           .98 1.05 1.11 1.12 1.03 1.06 1.09
+//   FP64 terrain 50   .90  .97 1.02 1.02  .93  .95  .99
+//   columns           21K  31K  38K  44K  53K  67K
+//   flat 80           .68  .78  .91 1.09 1.08 1.24
+//   flat 128          .59  .70  .81  .89 1.00  .98
+//   terrain 80        .79  .94 1.10 1.28 1.27 1.40
+//   terrain 128       .73  .85  .98 1.07 1.20 1.13
+//   precision 128     .78  .90 1.02 1.14 1.25 1.22
+//   FP64 100          .87 1.00 1.15 1.11 1.19 1.10
+//   FP64 terrain 100  .76  .89 1.04 1.00 1.07  .97
+// Flat, 3 levels 1.03 at 3 200 columns and 1.25 at 66 000; 6 levels .93 and
+// 1.15; 8 levels .97 at 39 000 and 1.12 at 66 000; 12 levels .99 there.
+// Ensembles of six members of 40 to 60 levels:
+//   columns           36K  44K  52K  62K  93K
+//   flat              .73  .76  .85  .92 1.00
+//   terrain           .75  .83  .90  .97 1.02
+//   precision         .79  .86  .92  .98 1.04
+//   FP64              .92  .98 1.01 1.06 1.05
+//   FP64 terrain      .88  .93  .98 1.04 1.00
+static int tile_columns(int nz, bool b3, bool prec, bool sums, bool many)
+{
+    const bool tall = nz > 64;
+    int k;
+    if (nz < 6) return 0;
+    if (ARW_F64) k = tall ? (b3 ? 36 : 30) : many ? (b3 ? 56 : 48) : (b3 ? 72 : 40);
+    else if (tall) k = b3 || prec ? 38 : 44;
+    else if (nz <= 40 || many) k = 72;
+    else k = b3 || prec ? 51 : sums ? 72 : 64;
+    if (nz < 12 && k > 40) k = 40;
+    return k * 1024;
+}
 
 // The tile's launch for nz levels: 16 columns keep a workgroup at 4 waves
 // (nz <= 64), four of them a CU at 112-120 VGPRs; 32 columns were slower
@@ -3280,7 +3318,8 @@ struct ColTile {
 };
 
 // false: k_column's domain, or more levels than a workgroup's 512 threads
-static bool column_tile(int cols, int nz, bool prec, ColTile& t)
+static bool column_tile(int cols, int nz, bool b3, bool prec, bool sums,
+                        bool many, ColTile& t)
 {
     const size_t tri = prec ? sizeof(double) : sizeof(real);
     constexpr int gpw = 64 / kTileX;
@@ -3291,7 +3330,7 @@ static bool column_tile(int cols, int nz, bool prec, ColTile& t)
     t.lds = (size_t)4 * (t.rows + 2 * TILE_PAD) * kTileX * tri
             + ((size_t)(t.rows + X_N * t.groups + 1) * kTileX + CF_N * t.rows)
                   * sizeof(real);
-    return cols <= kTileColumns && ng * kTileX <= 512;
+    return cols <= tile_columns(nz, b3, prec, sums, many) && ng * kTileX <= 512;
 }
 
 template <class SRC, bool B3, bool DAMP, bool AL, bool WW, bool PREC, bool XO>
@@ -3311,7 +3350,7 @@ static void launch_column(const Dom& d, const Sc& s0, real* pout,
                           hipStream_t st)
 {
     ColTile t;
-    if (column_tile(d.ny * d.nx, d.nz, s0.prec, t)) {
+    if (column_tile(d.ny * d.nx, d.nz, B3, s0.prec, WW, false, t)) {
         const dim3 g = tiles(d, kTileX);
         if (xo_active(d, s0))
             with_prec(s0.prec, [&](auto p) {
@@ -3506,7 +3545,7 @@ static void launch_column_b(const BatchSet& b, const Sc& s0, int cols,
     // for two steps when each group's 60 000 are tiled, 11.25 when none is
     ColTile t;
     const Batch& q = b.k[BK_TILE16];
-    if (column_tile(cols, q.nz, s0.prec, t)) {
+    if (column_tile(cols, q.nz, B3, s0.prec, false, true, t)) {
         with_prec(s0.prec, [&](auto p) {
             launch_column_tile<Many, B3, DAMP, AL, false, decltype(p)::value, true>(
                 q, bgrid(q), s0, nullptr, t, st);
@@ -3532,10 +3571,10 @@ static void launch_column_b_al(const BatchSet& b, const Sc& s, int al, int cols,
     else launch_column_b<B3, DAMP, false>(b, s, cols, st);
 }
 
-bool column_tiled(const BatchSet& b, bool prec, int cols)
+bool column_tiled(const BatchSet& b, bool b3, bool prec, int cols)
 {
     ColTile t;
-    return column_tile(cols, b.k[BK_TILE16].nz, prec, t);
+    return column_tile(cols, b.k[BK_TILE16].nz, b3, prec, false, true, t);
 }
 
 hipError_t run_column_b(const BatchSet& b, const Sc& s, bool b3, int write_al,
