@@ -195,10 +195,11 @@ __device__ __forceinline__ real flux3(real qm2, real qm1, real q0,
 //   x^GAMMA = x^2 s^3 x^e,  s = x^(-1/5), e = GAMMA - 7/5 = -2.4e-8,
 // s from the hardware's float log2/exp2 and one step of the series of
 // (1 - h)^(-1/5), h = 1 - x s^5 (|h| < 2e-5, next term 11/125 h^3 < 1e-15),
-// x^e from 1 + z + z^2/2, z = e ln x.  On [2^-16, 16] the error, mostly the
-// float logarithm's in z, stays below 512 double ulps, so a value at least
-// 1024 of them from a float rounding midpoint rounds as the exact one does;
-// the others (one in 2^18) and every other x take pow.
+// x^e from 1 + z + z^2/2, z = e ln x.  On [2^-16, 16] the error is mostly the
+// float logarithm's in z: at most 139 double ulps over every float there, 365
+// were the logarithm off by two ulps.  So a value at least 1024 of them from a
+// float rounding midpoint rounds as the exact one does; the others (one in
+// 2^18) and every other x take pow.
 __device__ __forceinline__ real pow_gamma(real x)
 {
 #if ARW_F64

@@ -30,3 +30,30 @@ def test_pressure_is_the_rounded_power():
     assert x.min() < 0.0 and x[x > 0.0].min() < 2.0 ** -16 and x.max() > 16.0
     assert np.array_equal(p, want, equal_nan=True), \
         np.flatnonzero(~((p == want) | (np.isnan(p) & np.isnan(want))))[:8]
+
+
+def test_pressure_over_whole_binades():
+    """2^23 arguments in each binade the short form takes, near every float
+    in it (no base theta, so theta' sets the argument to a rounding or two)."""
+    import torch
+    from arwen_amd import cases as C
+    from arwen_amd import dycore
+    from arwen_amd.state import DomainState
+    g = DomainState.from_host(C.ensemble_member(1024, 1024, 8, seed=3))
+    g.thb.zero_()
+    dycore.update_diagnostics(g)
+    p0alt = (g.alt.double() * 1.0e5).float().double()
+    m = torch.arange(1 << 23, device=g.alt.device).reshape(g.alt.shape)
+    gamma = float(np.float32(1.4))
+    for e in range(-16, 5):
+        target = (1.0 + m.double() * 2.0 ** -23) * 2.0 ** e
+        th = (target * p0alt / 287.0).float()
+        g.thp.copy_(th)
+        dycore.update_diagnostics(g)
+        # a double quotient of floats, rounded, is the float quotient
+        x = ((th.double() * 287.0).float().double() / p0alt).float()
+        want = (torch.pow(x.double(), gamma).float().double() * 1.0e5).float()
+        assert torch.equal(g.p, want), (e, int((g.p != want).sum()))
+        d = torch.unique(x).numel()
+        print(f"2^{e}: {d} arguments", flush=True)
+        assert d > 1 << 22
