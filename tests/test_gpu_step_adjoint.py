@@ -137,6 +137,41 @@ def test_stage_factors_and_flags_equal_plain_calls():
         assert torch.equal(a_new[n], a_ref[n]), n
 
 
+@pytest.mark.parametrize("dtype,nz", [
+    (torch.float64, 128), (torch.float64, 319), (torch.float64, 320),
+    (torch.float32, 639), (torch.float32, 640)])
+def test_stage_factors_of_many_levels_equal_plain_calls(dtype, nz):
+    """The sweeps over the stage's factors keep their rows in LDS, up to
+    160 KB (319 levels in FP64, 639 in FP32); more levels form the factors
+    anew.  Bit for bit the call without factors on both sides."""
+    from arwen_amd import adjoint, dycore
+    from arwen_amd.state import DomainState
+    from tests.helpers import random_state_case
+    case, rng = random_state_case(seed=6, nz=nz, ny=3, nx=7, hill=300.0)
+    # layers of 122 m2/s2 at 640 levels: noise of 20 would turn some over
+    case.fields["php"] *= 0.1
+    cfg, dtau = case.cfg, 0.5
+    print(f"stage factors {dtype} nz={nz}", flush=True)
+    g = DomainState.from_host(case, dtype=dtype)
+    dycore.update_diagnostics(g)
+    dycore.prepare_acoustic_coefficients(g, cfg, dtau)
+    for n in adjoint.ACOUSTIC_STATE:
+        a = getattr(g, n)
+        a.copy_(torch.as_tensor(0.05 * rng.standard_normal(a.shape)))
+    lam = {n: torch.as_tensor(rng.standard_normal(getattr(g, n).shape)).to(g.u)
+           for n in NAMES_OUT}
+    outs, accs = [], []
+    for lu in (None, adjoint.adjoint_factors(g, cfg, dtau)):
+        accs.append(adjoint.reference_accumulators(g))
+        outs.append(adjoint.acoustic_substep_adjoint(g, cfg, dtau, False, lam,
+                                                     accs[-1], lu=lu))
+    for n in outs[0]:
+        assert bool(torch.isfinite(outs[0][n]).all()), n
+        assert torch.equal(outs[0][n], outs[1][n]), n
+    for n in adjoint.ACOUSTIC_REF:
+        assert torch.equal(accs[0][n], accs[1][n]), n
+
+
 def test_set_w_surface_adjoint_matches_oracle():
     from arwen_amd import adjoint
     o, coefs, dtau, cfg, rng, g = _device_pair(hill=300.0)
