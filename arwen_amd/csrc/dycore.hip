@@ -1486,7 +1486,7 @@ int32_t substep(const Dom& d, const Sc& s, real* pout, int write_al,
                     KID_COLUMN, st);
 }
 
-// Up to this many columns the limiter runs thread per point on stored fluxes
+// Below this many columns the limiter runs thread per point on stored fluxes
 // (its column marches recompute every flux twice and end in a copy): 40x36x30
 // 315 us a step against 327, 96x100x40 with six species 591 against 606; but
 // 192x160x50 1016 against 988, 400x380x50 with ten species 8062 against 6953.

@@ -108,10 +108,11 @@ def test_microphysics_slot_runs_after_the_dynamics():
 
 @pytest.mark.parametrize("opt", [1, 0])
 def test_column_march_scalars_match_oracle_bitwise(opt):
-    """At 512 x 512 columns and more the step's scalar transport runs as
-    column marches (k_scalar_cols, and k_pd_scale_cols / k_pd_apply_cols
-    on the final stage); below it, one thread per point.  One WSM6 step at
-    that size against the oracle, with and without the PD limiter."""
+    """The step's unlimited scalar transport is a column march
+    (k_scalar_cols); from 128 x 128 columns on so is the final stage's limiter
+    (k_pd_scale_cols / k_pd_apply_cols), below it one thread per point.  One
+    WSM6 step at 512 x 512 columns against the oracle, with and without the PD
+    limiter."""
     from arwen_amd import dycore
     case = cases.mixed_phase(6, nx=512, ny=512, nz=6, dx=3000.0,
                              moist_adv_opt=opt)
