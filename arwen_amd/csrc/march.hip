@@ -3091,25 +3091,32 @@ static void launch_finish(const typename SRC::Arg& a, dim3 g,
 }
 
 // The held-mixing variants: one domain, plain form (arw_step's held
-// tendencies refuse the precision form and the ensemble).
+// tendencies refuse the precision form and the ensemble).  Without the step
+// options where none is live: 1000x1000x50 k_tend_cols 1308 -> 1110 us a launch,
+// k_tend_faces 1109 -> 1029 (the level groups had cost them 80 and 20).
 template <bool B3, bool DIFF>
 static void launch_tend_faces_held(const Dom& d, dim3 g, const Sc& s,
                                    hipStream_t st)
 {
-    hipLaunchKernelGGL((k_tend_faces<One, B3, DIFF, false, true>), g,
-                       dim3(64, 4), kTendFacesLds, st, d, s);
+    with_xo(xo_active(d, s), [&](auto xo) {
+        hipLaunchKernelGGL((k_tend_faces<One, B3, DIFF, false, true, decltype(xo)::value>),
+                           g, dim3(64, 4), kTendFacesLds, st, d, s);
+    });
 }
 
 template <bool B3, bool DIFF>
 static void launch_tend_cols_held(const Dom& d, dim3 g, const Sc& s,
                                   hipStream_t st)
 {
-    if (d.qv)
-        hipLaunchKernelGGL((k_tend_cols<One, B3, DIFF, true, false, true>), g,
-                           dim3(64, 4), 0, st, d, s);
-    else
-        hipLaunchKernelGGL((k_tend_cols<One, B3, DIFF, false, false, true>), g,
-                           dim3(64, 4), 0, st, d, s);
+    with_xo(xo_active(d, s), [&](auto xo) {
+        constexpr bool X = decltype(xo)::value;
+        if (d.qv)
+            hipLaunchKernelGGL((k_tend_cols<One, B3, DIFF, true, false, true, X>), g,
+                               dim3(64, 4), 0, st, d, s);
+        else
+            hipLaunchKernelGGL((k_tend_cols<One, B3, DIFF, false, false, true, X>), g,
+                               dim3(64, 4), 0, st, d, s);
+    });
 }
 
 // The stencil marches (k_tend_faces, k_tend_cols, the scalar kernels): a group
