@@ -54,6 +54,8 @@ def test_eager_ensemble_matches_member_steps_bitwise(terrain):
     _assert_same(seq, ens_states)
 
 
+# (these few columns are solved in tiles of 16 whatever col_tile says;
+# test_column_march_ensemble_matches_member_steps_bitwise reaches 64 and 128)
 @pytest.mark.parametrize("groups,order,join,tile", [
     (1, None, 0, 256), (2, "largest_first", 0, 128),
     (3, "smallest_first", 1, 64)])
